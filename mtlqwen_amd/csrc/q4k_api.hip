@@ -333,6 +333,11 @@ Workspace& workspace(int device) {
   return g_ws[device & 63];
 }
 
+bool stream_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
 // Device allocation for workspace growth.  hipMalloc is not allowed while a
 // stream captures a graph, and a failure there would look like a lack of
 // memory: a call on a capturing stream that needs more workspace than the
@@ -342,8 +347,7 @@ Workspace& workspace(int device) {
 std::atomic<uint64_t> g_ws_allocations{0};
 
 int ws_alloc(hipStream_t stream, int device, void** p, size_t bytes, const char* what) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone)
+  if (stream_capturing(stream))
     return fail(Q4K_ECAPTURE,
                 "the %s must grow to %zu bytes on device %d, but the stream is capturing a graph and allocation is not allowed "
                 "there: make one call of this shape (or a larger one) before the capture",
@@ -491,6 +495,36 @@ int set_device(int device) {
   return Q4K_OK;
 }
 
+// A prefill GEMM of the middle row counts (mid_plan): x staged as for the
+// other GEMMs, the K-slices' sums in the split-K workspace.  A capture that
+// finds the workspace too small takes one slice (no sums to hold) instead of
+// growing it.
+int run_mid(hipStream_t stream, Workspace& ws, q4k_weight* w, const GemmArgs& g, uint32_t dtype, MidPlan plan, bool gated) {
+  if (plan.slices > 1 && ws.part_elems < plan.part_floats && stream_capturing(stream))
+    plan.slices = 1;
+  if (plan.slices > 1) {
+    int rc = ensure_buffer(stream, ws, w->device, ws.part, ws.part_elems, plan.part_floats, "split-K workspace");
+    if (rc)
+      return rc;
+  }
+  MidArgs a;
+  a.w = g.w;
+  a.wu = g.wu;
+  a.xh = g.xh;
+  a.rowscale = g.rowscale;
+  a.y = g.y;
+  a.aux = g.aux;
+  a.part = ws.part;
+  a.m = g.m;
+  a.n = g.n;
+  a.nb = g.nb;
+  a.post = g.post;
+  a.dtype = (int)dtype;
+  LaunchTimer timer(stream, Q4K_KERNEL_GEMM);
+  Q4K_TRY_HIP(launch_mid(stream, a, w->type, plan, gated), "mid gemm launch");
+  return Q4K_OK;
+}
+
 // One projection (phase already chosen) on the weight's device, with the
 // device's workspace lock held.  restage == false reuses the staged x of the
 // previous call, which must have been a projection of the same x with the
@@ -528,6 +562,9 @@ int run_typed_gemm_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, cons
   a.k = (int)w->k;
   a.nb = (int)(w->k / 256);
   a.post = (int)post;
+  const MidPlan mid = mid_plan(a.m, a.n, a.nb, device_cus(w->device));
+  if (mid.rt)
+    return run_mid(stream, ws, w, a, dtype, mid, false);
   LaunchTimer timer(stream, Q4K_KERNEL_GEMM);
   Q4K_TRY_HIP(launch_typed_gemm(stream, a, w->type, (int)dtype, device_cus(w->device)), "typed gemm launch");
   return Q4K_OK;
@@ -757,6 +794,9 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
     a.k = (int)w->k;
     a.nb = (int)(w->k / 256);
     a.post = (int)post;
+    const MidPlan mid = mid_plan(a.m, a.n, a.nb, device_cus(w->device));
+    if (mid.rt)
+      return run_mid(stream, ws, w, a, dtype, mid, false);
     rc = gemm2_split_buffers(stream, ws, w->device, a, false);
     if (rc)
       return rc;
@@ -1212,6 +1252,9 @@ int mlp_gate_up_impl(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x
     a.k = (int)wg->k;
     a.nb = (int)(wg->k / 256);
     a.post = Q4K_POST_GATE;
+    const MidPlan mid = mid_plan(a.m, a.n, a.nb, device_cus(wg->device));
+    if (mid.rt)
+      return run_mid(s, ws, wg, a, dtype, mid, true);
     rc = gemm2_split_buffers(s, ws, wg->device, a, true);
     if (rc)
       return rc;

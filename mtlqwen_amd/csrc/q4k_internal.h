@@ -352,6 +352,19 @@ struct GemmArgs {
   int split_b = 0, split_q = 0;
 };
 
+struct MidArgs {
+  const uint8_t* w = nullptr;
+  const uint8_t* wu = nullptr;  // up weights of the gated form (w is the gate)
+  const _Float16* xh = nullptr; // staged activations in the GEMM order
+  const float* rowscale = nullptr;
+  void* y = nullptr;
+  const void* aux = nullptr;
+  float* part = nullptr;  // slice sums (slices > 1)
+  int m = 0, n = 0, nb = 0, post = 0, dtype = 0;
+  int slices = 1;                // K-slices
+  int cblocks = 0, rblocks = 0;  // set by the launch
+};
+
 struct GatherIndex {
   uint32_t rows;
   uint32_t src[64];
@@ -454,6 +467,20 @@ hipError_t launch_gemm2(hipStream_t s, const GemmArgs& a, int dtype, int cus);
 // same n and k, x staged once): y = SiLU(x W^T) * (x Wu^T) with the
 // roundings of the two-call form (gate stored, then up with post 2 over it).
 hipError_t launch_gemm2_gated(hipStream_t s, const GemmArgs& a, int dtype, int cus);
+
+// The plan of a prefill GEMM of the middle row counts (q4k_mid.hip): row tiles
+// per workgroup (0: not this form), K-slices, and the floats their sums take
+// in the split-K workspace (slices > 1).
+struct MidPlan {
+  int rt = 0, slices = 1;
+  size_t part_floats = 0;
+};
+constexpr int kMidMaxSlices = 16;
+constexpr size_t kMidPartFloats = 16u << 20;  // 64 MiB, the split-K partials of the no-allocation scratch
+MidPlan mid_plan(int m, int n, int nb, int cus);
+// x staged in the GEMM order; gated: SiLU(x W^T) * (x Wu^T) (Q4_K) with the
+// roundings of the two-call form.
+hipError_t launch_mid(hipStream_t s, MidArgs a, uint32_t type, const MidPlan& plan, bool gated);
 
 // One MFMA-ceiling launch: `blocks` workgroups of 4 waves, each wave issuing
 // 32 * iters v_mfma_f32_16x16x32_f16 (16384 FLOP each); out holds blocks * 256 floats.
