@@ -356,6 +356,7 @@ struct MidArgs {
   const uint8_t* w = nullptr;
   const uint8_t* wu = nullptr;  // up weights of the gated form (w is the gate)
   const _Float16* xh = nullptr; // staged activations in the GEMM order
+  const _Float16* xs = nullptr; // sub-block sums (hi/lo rows)
   const float* rowscale = nullptr;
   void* y = nullptr;
   const void* aux = nullptr;
@@ -396,6 +397,10 @@ enum StageMode : int {
 // k + eps) * norm_w (native_ops.metal:6-40), before the conversion.
 hipError_t launch_stage_x(hipStream_t s, const void* x, int dtype, _Float16* xo, _Float16* xs, float* rowscale, int m, int k, int mode,
                           const float* norm_w = nullptr, float eps = 0.0f);
+// The GEMM order (kStageGemm) with one row per workgroup, for few rows; xs:
+// hi/lo rows and the sub-block sums (stage_row_kernel).
+hipError_t launch_stage_rows(hipStream_t s, const void* x, int dtype, _Float16* xo, float* rowscale, int m, int k, const float* norm_w, float eps,
+                             _Float16* xs = nullptr);
 hipError_t launch_stage_pack(hipStream_t s, const void* x, int dtype, const DecodePack& pk, int m, int k);
 
 // Halves of the sub-block-sum fragments for `rows` staged rows: per 16-row
@@ -480,7 +485,13 @@ constexpr size_t kMidPartFloats = 16u << 20;  // 64 MiB, the split-K partials of
 MidPlan mid_plan(int m, int n, int nb, int cus);
 // x staged in the GEMM order; gated: SiLU(x W^T) * (x Wu^T) (Q4_K) with the
 // roundings of the two-call form.
+hipError_t launch_mid_reduce(hipStream_t s, const MidArgs& a, bool gated);
 hipError_t launch_mid(hipStream_t s, MidArgs a, uint32_t type, const MidPlan& plan, bool gated);
+
+// 1..64 rows staged as hi/lo pairs (launch_stage_rows with xs): y = post(x W^T)
+// or SiLU(x W^T) * (x Wu^T) with the decode GEMVs' precision, every weight
+// type; a.slices K-slices.
+hipError_t launch_rows_gemm(hipStream_t s, const MidArgs& a, uint32_t type, bool gated, int cus);
 
 // One MFMA-ceiling launch: `blocks` workgroups of 4 waves, each wave issuing
 // 32 * iters v_mfma_f32_16x16x32_f16 (16384 FLOP each); out holds blocks * 256 floats.

@@ -3307,6 +3307,13 @@ hipError_t launch_stage_x(hipStream_t s, const void* x, int dtype, _Float16* xo,
                           const float* norm_w, float eps) {
   if (m <= 0)
     return hipSuccess;
+  // One row per workgroup while 8 rows per workgroup leave CUs idle (fp32 /
+  // fp16, one row against eight: K = 4096, M = 128 3.2 / 3.3 against 5.4 /
+  // 7.2 us, M = 1024 7.5 / 7.8 against 7.6 / 12.4; K = 12288, M = 128 4.8 /
+  // 4.9 against 12.8 / 14.3, M = 1024 15.8 / 14.4 against 17.1 / 20.7; past
+  // that M = 2048 28.6 / 23.5 against 24.1 / 21.0).
+  if (mode == kStageGemm && m <= 1024)
+    return launch_stage_rows(s, x, dtype, xo, rowscale, m, k, norm_w, eps);
   RowNorm nrm;
   nrm.w = norm_w;
   nrm.eps = eps;

@@ -7,9 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 
-#include <type_traits>
-
-#include "q4k_formats.h"
+#include "q4k_mid.h"
 
 namespace q4k {
 namespace {
@@ -33,109 +31,6 @@ struct MidShape {
   static_assert(KG == 1 || 8 * (RT / 2) * CT * 1024 <= kLds, "K-group exchange");
 };
 
-// Load accounting.  A wave issues A(t + AD) (LA loads) at step t, then, at
-// odd steps t = 2 b + 1, its share of B(b + NB) (LB loads); the prologue
-// issues B(0), A(0 .. AD - 1), B(1 .. NB - 1).  At the top of step t A(t) must
-// have landed and, at odd steps, B((t + 1) / 2) (read from there on).  vmcnt
-// counts in issue order, so the wait is the number of loads issued after the
-// later of the two: the smallest over the steps of one parity, the first ones
-// (whose loads come from the prologue) included.
-constexpr int mid_loads_after(int t, int ad, int nb, int la, int lb) {
-  // Position of the last required load, and of the end, counted in loads.
-  int pos = lb, need = 0;  // after B(0)
-  for (int i = 0; i < ad; ++i) {
-    pos += la;
-    if (i == t + 1)
-      need = pos;
-  }
-  for (int b = 1; b < nb; ++b) {
-    pos += lb;
-    if ((t & 1) && b == (t + 1) / 2)
-      need = pos > need ? pos : need;
-  }
-  for (int s = 0; s < t; ++s) {
-    pos += la;
-    if (s + ad == t + 1)
-      need = pos > need ? pos : need;
-    if (s & 1) {
-      pos += lb;
-      if ((t & 1) && (s - 1) / 2 + nb == (t + 1) / 2)
-        need = pos > need ? pos : need;
-    }
-  }
-  return pos - need;
-}
-constexpr int mid_wait_count(int parity, int ad, int nb, int la, int lb) {
-  int n = 63;
-  for (int t = parity; t < 32; t += 2) {
-    const int v = mid_loads_after(t, ad, nb, la, lb);
-    n = v < n ? v : n;
-  }
-  return n;
-}
-
-template <int N>
-__device__ __forceinline__ void mid_wait() {
-  static_assert(N >= 0 && N < 64, "vmcnt field");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-template <typename OutT>
-__device__ __forceinline__ void mid_store(const MidArgs& a, int row, size_t col, float v, float rs) {
-  OutT* y = reinterpret_cast<OutT*>(a.y);
-  const size_t off = (size_t)row * a.n + col;
-  float acc_v = v * rs;
-  if (sizeof(OutT) == 2)
-    acc_v = round_half(acc_v);
-  float out = acc_v;
-  if (a.post == 1)
-    out = acc_v + load_elem(reinterpret_cast<const OutT*>(a.aux), off);
-  else if (a.post == 2)
-    out = silu(load_elem(reinterpret_cast<const OutT*>(a.aux), off)) * acc_v;
-  asm("" : "+v"(out));  // the fp32 value first: fused into the conversion the product would round once instead of twice
-  store_elem(y, off, out);
-}
-
-template <typename OutT>
-__device__ __forceinline__ void mid_store_gated(const MidArgs& a, int row, size_t col, float gv, float uv, float rs) {
-  OutT* y = reinterpret_cast<OutT*>(a.y);
-  gv *= rs;
-  uv *= rs;
-  if (sizeof(OutT) == 2) {
-    gv = round_half(gv);
-    uv = round_half(uv);
-  }
-  float out = silu(gv) * uv;
-  asm("" : "+v"(out));
-  store_elem(y, (size_t)row * a.n + col, out);
-}
-
-// Epilogue of the rows of one 16 x 16 accumulator tile (row tile rt0, output
-// column tile ct): lane 16g + i holds rows 4g .. 4g + 3 of column i.
-template <bool GATED>
-__device__ __forceinline__ void mid_epilogue_tile(const MidArgs& a, int rt0, int ct, int lane, const f4_t& v, const f4_t& up) {
-  const int row0 = 16 * rt0 + 4 * (lane >> 4);
-  const size_t col = (size_t)ct * 16 + (lane & 15);
-  const f4_t rs = *reinterpret_cast<const f4_t*>(a.rowscale + row0);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int row = row0 + e;
-    if (row >= a.m)
-      continue;
-    if constexpr (GATED) {
-      if (a.dtype == kF32)
-        mid_store_gated<float>(a, row, col, v[e], up[e], rs[e]);
-      else
-        mid_store_gated<_Float16>(a, row, col, v[e], up[e], rs[e]);
-    } else {
-      if (a.dtype == kF32)
-        mid_store<float>(a, row, col, v[e], rs[e]);
-      else
-        mid_store<_Float16>(a, row, col, v[e], rs[e]);
-    }
-  }
-}
-
 // The steps of one wave of K-group KGI (compile-time, so that the u-steps and
 // with them the dequantisation's shifts are).
 template <class P, int RT, int CT, int KG, int NS, int NB, bool GATED, int KGI>
@@ -147,7 +42,7 @@ __device__ __forceinline__ void mid_steps(const MidArgs& a, uint8_t* lds, int by
   constexpr int MB = KG == 1 ? CT : CT % 2 == 0 ? CT / 2 : KGI == 0 ? CT : 0;
   constexpr int MB0 = KG == 2 && CT % 2 == 0 ? KGI * (CT / 2) : 0;
   constexpr int LA = RT / 2, LB = MB * P::kNL;
-  constexpr int W0 = mid_wait_count(0, AD, NB, LA, LB), W1 = mid_wait_count(1, AD, NB, LA, LB);
+  constexpr int W0 = mid_wait_count(0, 1, AD, NB, LA, LB), W1 = mid_wait_count(1, 1, AD, NB, LA, LB);
   const int cg = KG == 1 ? wave : wave & 3, ntiles = a.n >> 4, steps = 2 * nbr;
   const int ct0 = (cb * M::kCG + cg) * OT;
   const uint8_t* wcol[MB > 0 ? MB : 1];
@@ -392,7 +287,162 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < OT; ++c)
       if (row_tile + h < live && ct0 + c < ntiles)
-        mid_epilogue_tile<GATED>(a, row_tile + h, ct0 + c, lane, sum[h][c], sum[h][GATED ? OT + c : c]);
+        mid_epilogue_tile<GATED>(a, row_tile + h, ct0 + c, lane, sum[h][c], sum[h][GATED ? OT + c : c], mid_rowscale(a, row_tile + h, lane));
+}
+
+// Activations of few rows in the GEMM order: one row per workgroup of 512
+// threads, so that a pass of 128 rows uses 128 CUs (8 rows per workgroup use
+// 16).  Workgroup L runs on XCD L % 8: the 8 rows that share each 128-byte
+// line of the staged operand go to one XCD, whose L2 puts the line together.
+// CPT chunks of 8 elements per thread stay in registers between the row
+// maximum (and, with NORM, the sum of squares) and the conversion; CPT == 0:
+// x is read twice.
+// SPLIT: a row is staged as two, hi = fp16(v) as staged row 32 (r / 16) +
+// r % 16 and lo = fp16(v - hi) 16 rows on (about 22 significant bits), and xs
+// receives each 32-element sub-block's sum / 32, hi/lo too, as the A operand
+// of v_mfma_f32_16x16x16_f16 per (block, row tile): lane 16 G + r % 16 holds
+// sub-blocks 4 (G & 1) .. + 3, the low parts for G >= 2.
+template <typename InT, int CPT, bool NORM, bool SPLIT>
+__global__ __launch_bounds__(512) void stage_row_kernel(const InT* __restrict__ x, _Float16* __restrict__ xo, float* __restrict__ rowscale, int m,
+                                                        int k, const float* __restrict__ nw, float eps, _Float16* __restrict__ xs) {
+  constexpr int T = 512, N = CPT > 0 ? CPT : 1;
+  const int j8 = (int)blockIdx.x >> 3, row = ((j8 >> 3) * 8 + ((int)blockIdx.x & 7)) * 8 + (j8 & 7);
+  if (row >= m)
+    return;
+  const int tid = threadIdx.x, chunks = k >> 3, nb = k >> 8;
+  const InT* xr = x + (size_t)row * k;
+  float v[N][8];
+  float mx = 0.0f, ss = 0.0f;
+  auto read = [&](int c, float (&o)[8]) {
+    load8(xr + (size_t)c * 8, o);
+    if (NORM) {
+      float w8[8];
+      load8(nw + (size_t)c * 8, w8);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        ss = fmaf(o[i], o[i], ss);
+        o[i] *= w8[i];
+      }
+    }
+  };
+  if constexpr (CPT > 0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int c = tid + T * j;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        v[j][i] = 0.0f;
+      if (c < chunks)
+        read(c, v[j]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        mx = fmaxf(mx, fabsf(v[j][i]));
+    }
+  } else {
+    for (int c = tid; c < chunks; c += T) {
+      read(c, v[0]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        mx = fmaxf(mx, fabsf(v[0][i]));
+    }
+  }
+  __shared__ float red[2][8];
+  mx = max64_lanes(mx);
+  if (NORM) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      ss += __shfl_xor(ss, off);
+  }
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = mx;
+    red[1][tid >> 6] = ss;
+  }
+  __syncthreads();
+  ss = 0.0f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    mx = fmaxf(mx, red[0][w]);
+    ss += red[1][w];
+  }
+  float r = 1.0f;
+  if (NORM) {
+    r = 1.0f / sqrtf(ss / (float)k + eps);
+    mx *= r;
+  }
+  float up, down;
+  pow2_scale(mx, up, down);
+  if (tid == 0)
+    rowscale[row] = down;
+  const float cs = NORM ? up * r : up;
+  // Whole groups of 4 lanes (one sub-block) call it together.
+  auto put = [&](int c, const float (&o)[8]) {
+    h8_t h;
+    if constexpr (SPLIT) {
+      h8_t lo;
+      float sum = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        // One fp32 value for both parts: fused into the conversions, hi would
+        // be rounded once where it is stored and its residual taken from
+        // another rounding of the product (cs is no power of two with NORM).
+        float t = o[i] * cs;
+        asm("" : "+v"(t));
+        h[i] = (_Float16)t;
+        lo[i] = (_Float16)(t - (float)h[i]);
+        sum += t;
+      }
+      const int vrow = 32 * (row >> 4) + (row & 15);
+      *reinterpret_cast<h8_t*>(xo + gemm_frag_offset(vrow, c, nb)) = h;
+      *reinterpret_cast<h8_t*>(xo + gemm_frag_offset(vrow + 16, c, nb)) = lo;
+      sum += dpp_f<kDppQuadSwap1>(sum);
+      sum += dpp_f<kDppQuadSwap2>(sum);
+      if ((c & 3) == 0) {
+        const float s32 = sum * 0.03125f;
+        const _Float16 sh = (_Float16)s32;
+        const int jb = (c >> 2) & 7;
+        _Float16* p = xs + (((size_t)(c >> 5) * ((m + 15) >> 4) + (row >> 4)) * 64 + 16 * (jb >> 2) + (row & 15)) * 4 + (jb & 3);
+        p[0] = sh;
+        p[128] = (_Float16)(s32 - (float)sh);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        h[i] = (_Float16)(o[i] * cs);
+      *reinterpret_cast<h8_t*>(xo + gemm_frag_offset(row, c, nb)) = h;
+    }
+  };
+  if constexpr (CPT > 0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int c = tid + T * j;
+      if (c < chunks)
+        put(c, v[j]);
+    }
+  } else {
+    for (int c = tid; c < chunks; c += T) {
+      read(c, v[0]);
+      put(c, v[0]);
+    }
+  }
+}
+
+template <typename InT, bool NORM, bool SPLIT>
+void stage_rows(hipStream_t s, const InT* x, _Float16* xo, float* rowscale, int m, int k, const float* nw, float eps, _Float16* xs) {
+  const dim3 grid((unsigned)((m + 63) / 64 * 64)), block(512);
+  if (k <= 4096)
+    (void)dispatch(stage_row_kernel<InT, 1, NORM, SPLIT>, grid, block, s, x, xo, rowscale, m, k, nw, eps, xs);
+  else if (k <= 12288)
+    (void)dispatch(stage_row_kernel<InT, 3, NORM, SPLIT>, grid, block, s, x, xo, rowscale, m, k, nw, eps, xs);
+  else
+    (void)dispatch(stage_row_kernel<InT, 0, NORM, SPLIT>, grid, block, s, x, xo, rowscale, m, k, nw, eps, xs);
+}
+
+template <typename InT>
+void stage_rows_any(hipStream_t s, const InT* x, _Float16* xo, float* rowscale, int m, int k, const float* nw, float eps, _Float16* xs) {
+  if (xs)
+    nw ? stage_rows<InT, true, true>(s, x, xo, rowscale, m, k, nw, eps, xs) : stage_rows<InT, false, true>(s, x, xo, rowscale, m, k, nw, eps, xs);
+  else
+    nw ? stage_rows<InT, true, false>(s, x, xo, rowscale, m, k, nw, eps, xs) : stage_rows<InT, false, false>(s, x, xo, rowscale, m, k, nw, eps, xs);
 }
 
 // One wave per 16 x 16 output tile: the slices' sums in slice order, then the
@@ -413,7 +463,7 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(MidArgs a) {
     if (GATED)
       u += part[i * stride + (size_t)ntiles * 64];
   }
-  mid_epilogue_tile<GATED>(a, rt, ct, lane, s, u);
+  mid_epilogue_tile<GATED>(a, rt, ct, lane, s, u, mid_rowscale(a, rt, lane));
 }
 
 template <class P, int RT, int CT, bool GATED>
@@ -435,8 +485,7 @@ hipError_t mid_launch(hipStream_t s, MidArgs a) {
   (void)dispatch(mid_gemm_kernel<P, RT, CT, KG, NS, NB, GATED>, dim3((unsigned)grid), dim3(512), s, a);
   if (a.slices > 1) {
     dispatch_events() = DispatchEvents{nullptr, ev.stop};
-    const int items = (a.m + 15) / 16 * ntiles;
-    (void)dispatch(mid_reduce_kernel<GATED>, dim3((unsigned)((items + 3) / 4)), dim3(256), s, a);
+    (void)launch_mid_reduce(s, a, GATED);
     dispatch_events() = ev;
   }
   return hipGetLastError();
@@ -500,6 +549,24 @@ MidPlan mid_plan(int m, int n, int nb, int cus) {
   }
   p.part_floats = p.slices > 1 ? p.slices * row_floats : 0;
   return p;
+}
+
+hipError_t launch_stage_rows(hipStream_t s, const void* x, int dtype, _Float16* xo, float* rowscale, int m, int k, const float* norm_w, float eps,
+                             _Float16* xs) {
+  if (dtype == kF32)
+    stage_rows_any(s, static_cast<const float*>(x), xo, rowscale, m, k, norm_w, eps, xs);
+  else
+    stage_rows_any(s, static_cast<const _Float16*>(x), xo, rowscale, m, k, norm_w, eps, xs);
+  return hipGetLastError();
+}
+
+hipError_t launch_mid_reduce(hipStream_t s, const MidArgs& a, bool gated) {
+  const int items = (a.m + 15) / 16 * (a.n / 16);
+  if (gated)
+    (void)dispatch(mid_reduce_kernel<true>, dim3((unsigned)((items + 3) / 4)), dim3(256), s, a);
+  else
+    (void)dispatch(mid_reduce_kernel<false>, dim3((unsigned)((items + 3) / 4)), dim3(256), s, a);
+  return hipGetLastError();
 }
 
 hipError_t launch_mid(hipStream_t s, MidArgs a, uint32_t type, const MidPlan& plan, bool gated) {
