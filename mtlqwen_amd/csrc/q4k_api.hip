@@ -619,12 +619,81 @@ int run_gemv_groups_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, con
   return Q4K_OK;
 }
 
+// 9 to 63 rows of the other types (and of the wide Q4_K projections): x staged
+// once as hi/lo rows, then one GEMM over all rows with the group GEMV's
+// precision (rows_gemm_kernel), instead of one GEMV per 8 rows, each reading
+// the weights again: the Q6_K LM head (N = 248320) of 40 rows 262 us against
+// 803, the Q6_K / Q5_K 12288 -> 4096 projection of 19 rows 24 us against 66.
+// wu != nullptr: the fused gate/up pair (one type).
+constexpr uint32_t kRowsGemmMaxK = 32768;
+
+bool rows_gemm_fits(hipStream_t stream, const Workspace& ws, uint32_t m, uint32_t k, size_t part_floats) {
+  // A capture may not grow the workspace: it keeps the GEMV groups then.
+  return (ws.x_elems >= (size_t)128 * k + (size_t)4 * k && ws.scale && ws.part_elems >= part_floats) || ws.fixed || !stream_capturing(stream);
+}
+
+// K-slices that fill the CUs the column blocks leave idle, each at least two
+// blocks long.
+int rows_gemm_slices(uint32_t m, uint32_t n, uint32_t nb, bool gated, int cus) {
+  const int cblocks = (int)(gated ? (n / 16 + 3) / 4 : (n / 16 + 7) / 8);
+  int s = cus / cblocks < (int)nb / 2 ? cus / cblocks : (int)nb / 2;
+  s = s > kMidMaxSlices ? kMidMaxSlices : s;
+  const size_t row_floats = (size_t)((m + 15) / 16 * 16) * n * (gated ? 2 : 1);
+  while (s > 1 && s * row_floats > kMidPartFloats)
+    --s;
+  return s < 1 ? 1 : s;
+}
+
+int run_rows_gemm_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weight* wu, const void* x, void* y, const void* aux, uint32_t m,
+                         uint32_t post, uint32_t dtype, const float* norm_w, float eps) {
+  MidArgs a;
+  a.slices = rows_gemm_slices(m, w->n, w->k / 256, wu != nullptr, device_cus(w->device));
+  const size_t part = a.slices > 1 ? (size_t)a.slices * ((m + 15) / 16 * 16) * w->n * (wu ? 2 : 1) : 0;
+  // 128 staged rows, then the sub-block sums: 256 halves per block and row tile.
+  int rc = ensure_workspace(stream, ws, w->device, (size_t)128 * w->k + (size_t)4 * w->k, 64);
+  if (!rc && part)
+    rc = ensure_buffer(stream, ws, w->device, ws.part, ws.part_elems, part, "split-K workspace");
+  if (rc)
+    return rc;
+  _Float16* const xs = ws.x + (size_t)128 * w->k;
+  {
+    LaunchTimer timer(stream, Q4K_KERNEL_STAGE);
+    Q4K_TRY_HIP(launch_stage_rows(stream, x, (int)dtype, ws.x, ws.scale, (int)m, (int)w->k, norm_w, eps, xs), "stage_rows launch");
+  }
+  a.w = w->data;
+  a.wu = wu ? wu->data : nullptr;
+  a.xh = ws.x;
+  a.xs = xs;
+  a.rowscale = ws.scale;
+  a.y = y;
+  a.aux = aux;
+  a.part = ws.part;
+  a.m = (int)m;
+  a.n = (int)w->n;
+  a.nb = (int)(w->k / 256);
+  a.post = (int)post;
+  a.dtype = (int)dtype;
+  LaunchTimer timer(stream, wu ? Q4K_KERNEL_GEMV_GATED : Q4K_KERNEL_GEMV);
+  Q4K_TRY_HIP(launch_rows_gemm(stream, a, w->type, wu != nullptr, device_cus(w->device)), "rows gemm launch");
+  return Q4K_OK;
+}
+
+// Whether 9..63 rows of this weight (pair) take the rows GEMM now.
+bool rows_gemm_takes(hipStream_t stream, const Workspace& ws, const q4k_weight* w, uint32_t m, bool gated) {
+  if (m <= 8 || m >= kTypedGemmRows || w->k > kRowsGemmMaxK)
+    return false;
+  const int s = rows_gemm_slices(m, w->n, w->k / 256, gated, device_cus(w->device));
+  return rows_gemm_fits(stream, ws, m, w->k, s > 1 ? (size_t)s * ((m + 15) / 16 * 16) * w->n * (gated ? 2 : 1) : 0);
+}
+
 // Outputs narrower than kGemmMinColumns take the GEMV groups at every row
 // count, as with Q4_K (the per-row bar).
 int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const void* x, void* y, const void* aux, uint32_t m, uint32_t post,
                      uint32_t dtype, const float* norm_w, float eps) {
   if (m >= kTypedGemmRows && w->n >= kGemmMinColumns)
     return run_typed_gemm_locked(stream, ws, w, x, y, aux, m, post, dtype, norm_w, eps);
+  if (rows_gemm_takes(stream, ws, w, m, false))
+    return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   int rc = prenorm(stream, ws, w->device, x, norm_w, eps, m, w->k, dtype);
   if (rc)
     return rc;
@@ -644,6 +713,13 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
   Kernel& kern = resolve(w, phase);
   if (wu)
     resolve(wu, phase);
+  // Wide plain projections (the LM head) of 9 to 48 rows: the rows GEMM, whose
+  // rings run on across its column blocks (N = 248320, K = 4096: M = 16 151 us
+  // against 233 on the staged GEMV, 24 194 / 335, 32 200 / 241, 40 240 / 346).
+  // With fewer column blocks the staged and rows GEMVs are ahead (N = 4096, M
+  // = 40: 12.3 us against 17.6; N = 12288: 23.9 against 26.0).
+  if (!wu && m <= 16u * kGemvMaxRowTiles && (int)(w->n / 16) >= 16 * device_cus(w->device) && rows_gemm_takes(stream, ws, w, m, false))
+    return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   if (!wu && w->n < kGemmMinColumns && m > kGemvSplitRows) {
     int rc = prenorm(stream, ws, w->device, x, norm_w, eps, m, w->k, dtype);
     if (rc)
@@ -1227,6 +1303,11 @@ int mlp_gate_up_impl(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x
   }
   Workspace& ws = workspace(wg->device);
   std::lock_guard<std::mutex> lock(ws.mu);
+  if (!q4 && wg->type == wu->type && rows_gemm_takes(s, ws, wg, m, true)) {
+    resolve(wg, phase);
+    resolve(wu, phase);
+    return run_rows_gemm_locked(s, ws, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, norm_w, eps);
+  }
   if (q4 && resolve(wg, phase).kind == kGemm && m > 16u * kGemvMaxRowTiles && gemm2_supported((int)m, (int)wg->n)) {
     // Both projections on the pipelined GEMM: one gated launch over x staged
     // once computes SiLU(gate) * up with the two-call form's roundings (the
