@@ -1527,124 +1527,194 @@ constexpr int kGemmNarrowTileTime = 6;
 constexpr int kG2ASlot = 16 * 1024;                    // 8 row tiles x 2 fragments x 1 KB
 constexpr int kG2BWave = 2 * 4 * kTileBlockBytes;      // per wave: 2 blocks x 4 tile-blocks
 
-// Epilogue of a 128 x 64 wave tile.  Lane (col, g) holds rows 16 rt + 4 g + v
-// of column col of each column tile.  The aux loads (post 1 / 2) run one row
-// tile ahead of the stores: those of row tile rt + 1 are issued before the
-// stores of row tile rt, so their latency overlaps the previous tile's stores
-// instead of being paid once per row tile (rows differ, so an aux that is y
-// itself is read before it is written).  A tile wholly inside m (FULL) has no
-// per-row checks.  CT column tiles per wave, of which the first nct lie
-// inside n.
-template <typename OutT, int POST, bool FULL, int CT = 4>
-__device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, const f4_t (&acc)[8][CT], int mt0, int ct0, int lane, int nct = CT,
-                                               float* lrs = nullptr) {
+// Epilogues of a wave's 128-row tile.  The accumulators hold one column per
+// lane (4-byte pieces of 16 columns): stored as they are, the residual or gate
+// (aux) came in pieces of 32 or 64 bytes whose latency showed once per row
+// tile.  Each row tile therefore passes through the wave's own LDS (its B ring,
+// idle once its loads have landed: no barrier) and leaves as 4 consecutive
+// columns per lane, and the aux of a whole batch of row tiles is loaded, 4
+// columns per lane, before the first of them is stored.  N = 12288, K = 4096,
+// post 1, before and after: fp16 Q8_0 M = 1531 215 -> 184 us, M = 2048 270 ->
+// 231, Q6_K M = 2048 291 -> 249, Q4_K 256 -> 231, IQ4_XS 287 -> 265; fp32 Q8_0
+// 245 -> 233, Q6_K 263 -> 249 and, with six column tiles, Q4_K at M = 1531 223
+// -> 211, at M = 2048 242 -> 241.
+constexpr int kEpiLd(int cols) {
+  return cols + 4;  // floats per LDS row: the two row halves of a write fall in different banks
+}
+
+template <typename OutT>
+struct Quad;
+template <>
+struct Quad<float> {
+  typedef f4_t type;
+};
+template <>
+struct Quad<_Float16> {
+  typedef h4_t type;
+};
+
+// Four consecutive outputs (or aux values); vec: the pointer is aligned to them.
+template <typename OutT>
+__device__ __forceinline__ typename Quad<OutT>::type load_quad(const OutT* p, bool vec) {
+  typedef typename Quad<OutT>::type Q;
+  if (vec)
+    return *reinterpret_cast<const Q*>(p);
+  return Q{p[0], p[1], p[2], p[3]};
+}
+
+template <typename OutT>
+__device__ __forceinline__ void store_quad(OutT* p, typename Quad<OutT>::type v, bool vec) {
+  if (vec) {
+    *reinterpret_cast<typename Quad<OutT>::type*>(p) = v;
+  } else {
+    p[0] = v[0];
+    p[1] = v[1];
+    p[2] = v[2];
+    p[3] = v[3];
+  }
+}
+
+// LDS written by some lanes of a wave and read by others: the wave's LDS
+// accesses execute in order, and the fences keep the compiler from moving them
+// across this point (they emit no instruction at wavefront scope).
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// `value(rt, c, v)` forms the output (before aux) of accumulator element v of
+// row tile rt and output column tile c (of NC, nct of them inside n); wl is
+// wave-private LDS of at least 16 kEpiLd(16 NC) floats.
+template <typename OutT, int POST, int NC, int BR, typename F>
+__device__ __forceinline__ void gemm2_flush(const GemmArgs& a, float* wl, int mt0, int ct0, int lane, int nct, F value) {
+  typedef typename Quad<OutT>::type Q;
+  constexpr int LD = kEpiLd(16 * NC), LPR = 4 * NC, RPP = 64 / LPR, NP = (16 + RPP - 1) / RPP;  // lanes per row, rows per pass, passes
+  static_assert(8 % BR == 0, "batches of row tiles");
+  asm volatile("" : "+v"(lane));  // nothing of the epilogue is formed ahead of the K loop, beside its registers
   OutT* y = reinterpret_cast<OutT*>(a.y);
   const OutT* aux = reinterpret_cast<const OutT*>(a.aux);
   const int g = lane >> 4, col = lane & 15;
-  const int row0 = mt0 * 16 + 4 * g;
-  constexpr bool full = FULL;
-  // Row scales exist for the padded rows (the staging buffers cover whole
-  // 128-row tiles), so these 16-byte loads stay in bounds.
-  // Row scales of the 8 row tiles up front and the aux of row tile rt + 1
-  // loaded under the stores of row tile rt (two buffers).  With more than
-  // four column tiles per wave the registers of all that do not fit beside
-  // the six-tile loop's: the wave stages the tile's 128 row scales in its own
-  // LDS (lrs, its B ring, idle once its loads have landed) with one load and
-  // reads each row tile's from there, and loads each row tile's aux just
-  // before it.
-  constexpr bool ahead = CT <= 4;
-  f4_t rs[8];
-  if constexpr (ahead) {
+  const int lr = lane / LPR, lc = lane % LPR;
+  const bool live = lr < RPP && (lc >> 2) < nct;
+  const size_t col0 = (size_t)ct0 * 16 + 4 * lc;
+  const bool vec = ((reinterpret_cast<uintptr_t>(y) | (POST ? reinterpret_cast<uintptr_t>(aux) : 0)) & (4 * sizeof(OutT) - 1)) == 0;
 #pragma unroll
-    for (int rt = 0; rt < 8; ++rt)
-      rs[rt] = *reinterpret_cast<const f4_t*>(a.rowscale + row0 + 16 * rt);
-  } else {
-    *reinterpret_cast<float2*>(lrs + 2 * lane) = *reinterpret_cast<const float2*>(a.rowscale + mt0 * 16 + 2 * lane);
-  }
-  const size_t col0 = (size_t)ct0 * 16 + col;
-  float av[2][4][CT];
-  auto load_aux = [&](int rt, float (&dst)[4][CT]) {
+  for (int b = 0; b < 8; b += BR) {
+    Q av[POST ? BR : 1][NP];
+    if constexpr (POST != 0) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+      for (int r = 0; r < BR; ++r)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        const int row = row0 + 16 * rt + v;
-        dst[v][c] = (full || row < a.m) && c < nct ? load_elem(aux, (size_t)row * a.n + col0 + 16 * c) : 0.0f;
+        for (int p = 0; p < NP; ++p) {
+          const int lrow = p * RPP + lr, row = (mt0 + b + r) * 16 + lrow;
+          av[r][p] = Q{};
+          if (live && lrow < 16 && row < a.m)
+            av[r][p] = load_quad(aux + (size_t)row * a.n + col0, vec);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < BR; ++r) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+          wl[(4 * g + v) * LD + 16 * c + col] = value(b + r, c, v);
+      wave_order();
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        const int lrow = p * RPP + lr, row = (mt0 + b + r) * 16 + lrow;
+        if (live && lrow < 16 && row < a.m) {
+          const f4_t t = *reinterpret_cast<const f4_t*>(wl + lrow * LD + 4 * lc);
+          Q o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float out = t[e];
+            if constexpr (POST == 1)
+              out += (float)av[r][p][e];
+            if constexpr (POST == 2)
+              out *= silu((float)av[r][p][e]);
+            // The fp32 value is formed before any conversion to fp16: fused
+            // into the conversion (v_fma_mix) the product would round once
+            // instead of twice, as the reference's half(silu(g) * u) does.
+            asm("" : "+v"(out));
+            o[e] = (OutT)out;
+          }
+          store_quad(y + (size_t)row * a.n + col0, o, vec);
+        }
       }
-  };
-  if (POST != 0 && ahead)
-    load_aux(0, av[0]);
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
-    if (POST != 0 && ahead && rt + 1 < 8)
-      load_aux(rt + 1, av[(rt + 1) & 1]);
-    if (POST != 0 && !ahead)
-      load_aux(rt, av[0]);
-    if constexpr (!ahead)
-      rs[rt] = *reinterpret_cast<const f4_t*>(lrs + 16 * rt + 4 * g);
-    const float (&cur)[4][CT] = av[ahead ? rt & 1 : 0];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = row0 + 16 * rt + v;
-      if (!full && row >= a.m)
-        continue;
-#pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        if (c >= nct)
-          continue;
-        float acc_v = acc[rt][c][v] * rs[rt][v];
-        if (sizeof(OutT) == 2)
-          acc_v = round_half(acc_v);
-        float out = POST == 1 ? acc_v + cur[v][c] : POST == 2 ? silu(cur[v][c]) * acc_v : acc_v;
-        // The fp32 value is formed before any conversion to fp16: fused into
-        // the conversion (v_fma_mix) the product would round once instead of
-        // twice, as the reference's half(silu(g) * u) does.
-        asm("" : "+v"(out));
-        store_elem(y, (size_t)row * a.n + col0 + 16 * c, out);
-      }
+      wave_order();
     }
   }
 }
 
-// Epilogue of the gated GEMM's wave tile of 128 rows and CT / 2 output column
-// tiles: the gate tiles (columns 0 .. CT / 2 - 1 of acc) and the up tiles
-// (the rest) of the same output column tiles combine as in the two-call
-// form: SiLU(gate) * up, each of gate and up first unscaled and, for fp16
-// outputs, rounded to fp16 (the gate value the first call stores, the up
-// value the second call's epilogue forms).  nct of the output tiles lie
-// inside n.
-template <typename OutT, bool FULL, int CT = 4>
-__device__ __forceinline__ void gemm2_epilogue_gated(const GemmArgs& a, const f4_t (&acc)[8][CT], int mt0, int ct0, int lane, int nct) {
-  constexpr int H = CT / 2;  // output tiles: gate columns 0 .. H - 1, up columns H .. CT - 1
-  OutT* y = reinterpret_cast<OutT*>(a.y);
-  const int g = lane >> 4, col = lane & 15;
-  const int row0 = mt0 * 16 + 4 * g;
-  f4_t rs[8];
+// Row tiles whose aux is loaded together: as many as the registers hold (beside
+// six column tiles' accumulators one, and half its columns at a time).
+template <typename OutT, int CT>
+constexpr int epi_batch() {
+  return CT > 4 ? 1 : CT * sizeof(OutT) <= 16 ? 8 : 4;
+}
+
+template <typename OutT, int POST, int CT>
+__device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, const f4_t (&acc)[8][CT], int mt0, int ct0, int lane, int nct, float* wl) {
+  // The tile's 128 row scales behind the transposing buffer (the staging
+  // buffers cover whole 128-row tiles, so the loads stay in bounds).
+  float* const lrs = wl + 16 * kEpiLd(16 * CT);
+  *reinterpret_cast<float2*>(lrs + 2 * lane) = *reinterpret_cast<const float2*>(a.rowscale + mt0 * 16 + 2 * lane);
+  wave_order();
+  const int g = lane >> 4;
+  if constexpr (POST == 0) {
+    // Nothing to wait for: the pieces of 16 columns leave as they are (through
+    // LDS N = 12288, M = 2048 took 2 to 12 us more).
+    OutT* y = reinterpret_cast<OutT*>(a.y);
+    const size_t col0 = (size_t)ct0 * 16 + (lane & 15);
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-    rs[rt] = *reinterpret_cast<const f4_t*>(a.rowscale + row0 + 16 * rt);
-  const size_t col0 = (size_t)ct0 * 16 + col;
+    for (int rt = 0; rt < 8; ++rt) {
+      const f4_t rs = *reinterpret_cast<const f4_t*>(lrs + 16 * rt + 4 * g);
 #pragma unroll
-  for (int rt = 0; rt < 8; ++rt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = row0 + 16 * rt + v;
-      if (!FULL && row >= a.m)
-        continue;
-#pragma unroll
-      for (int c = 0; c < H; ++c) {
-        if (c >= nct)
+      for (int v = 0; v < 4; ++v) {
+        const int row = (mt0 + rt) * 16 + 4 * g + v;
+        if (row >= a.m)
           continue;
-        float gv = acc[rt][c][v] * rs[rt][v], uv = acc[rt][H + c][v] * rs[rt][v];
-        if (sizeof(OutT) == 2) {
-          gv = round_half(gv);
-          uv = round_half(uv);
-        }
-        float out = silu(gv) * uv;
-        asm("" : "+v"(out));  // the fp32 value first, as in the post-2 epilogue
-        store_elem(y, (size_t)row * a.n + col0 + 16 * c, out);
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          if (c < nct)
+            store_elem(y, (size_t)row * a.n + col0 + 16 * c, acc[rt][c][v] * rs[v]);
       }
     }
+  } else {
+    constexpr int NC = CT > 4 ? CT / 2 : CT;
+#pragma unroll
+    for (int c0 = 0; c0 < CT; c0 += NC)
+      gemm2_flush<OutT, POST, NC, epi_batch<OutT, CT>()>(a, wl, mt0, ct0 + c0, lane, nct - c0, [&](int rt, int c, int v) {
+        const float t = acc[rt][c0 + c][v] * lrs[16 * rt + 4 * g + v];
+        return sizeof(OutT) == 2 ? round_half(t) : t;
+      });
+  }
+}
+
+// The gated GEMM's wave tile of 128 rows and CT / 2 output column tiles: the
+// gate tiles (columns 0 .. CT / 2 - 1 of acc) and the up tiles (the rest) of
+// the same output column tiles combine as in the two-call form: SiLU(gate) *
+// up, each of gate and up first unscaled and, for fp16 outputs, rounded to
+// fp16 (the gate value the first call stores, the up value the second call's
+// epilogue forms).  nct of the output tiles lie inside n.
+template <typename OutT, int CT>
+__device__ __forceinline__ void gemm2_epilogue_gated(const GemmArgs& a, const f4_t (&acc)[8][CT], int mt0, int ct0, int lane, int nct, float* wl) {
+  constexpr int H = CT / 2;  // output tiles: gate columns 0 .. H - 1, up columns H .. CT - 1
+  float* const lrs = wl + 16 * kEpiLd(16 * H);
+  *reinterpret_cast<float2*>(lrs + 2 * lane) = *reinterpret_cast<const float2*>(a.rowscale + mt0 * 16 + 2 * lane);
+  wave_order();
+  const int g = lane >> 4;
+  gemm2_flush<OutT, 0, H, 8>(a, wl, mt0, ct0, lane, nct, [&](int rt, int c, int v) {
+    const float rs = lrs[16 * rt + 4 * g + v];
+    float gv = acc[rt][c][v] * rs, uv = acc[rt][H + c][v] * rs;
+    if (sizeof(OutT) == 2) {
+      gv = round_half(gv);
+      uv = round_half(uv);
+    }
+    return silu(gv) * uv;
+  });
 }
 
 // Tile order of the persistent GEMMs.  Workgroup b runs on XCD b % 8 (the
@@ -1980,20 +2050,20 @@ __device__ __forceinline__ void gemm2_tile(const GemmArgs& a, uint8_t* lds, int 
       reset_counter(ctr);  // ready for the next launch
   }
 
-  // One straight-line epilogue per (post code, tile inside m or not).
-  const bool full = mt0 * 16 + kG2M <= a.m;
+  // One straight-line epilogue per post code.
+  float* const elds = reinterpret_cast<float*>(bring);  // this wave's B ring: its loads have landed
   if constexpr (GATED) {
     const int nct2 = ntiles - ct0 >= 2 ? 2 : ntiles - ct0 > 0 ? ntiles - ct0 : 0;
-    full ? gemm2_epilogue_gated<OutT, true>(a, acc, mt0, ct0, lane, nct2) : gemm2_epilogue_gated<OutT, false>(a, acc, mt0, ct0, lane, nct2);
+    gemm2_epilogue_gated<OutT>(a, acc, mt0, ct0, lane, nct2, elds);
     return;
   }
   const int nct = ntiles - ct0 >= 4 ? 4 : ntiles - ct0 > 0 ? ntiles - ct0 : 0;
   if (a.post == 0)
-    full ? gemm2_epilogue<OutT, 0, true>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 0, false>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 0>(a, acc, mt0, ct0, lane, nct, elds);
   else if (a.post == 1)
-    full ? gemm2_epilogue<OutT, 1, true>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 1, false>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 1>(a, acc, mt0, ct0, lane, nct, elds);
   else
-    full ? gemm2_epilogue<OutT, 2, true>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 2, false>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 2>(a, acc, mt0, ct0, lane, nct, elds);
 }
 
 // Persistent launch: workgroup b takes its tiles in the order of the tile
@@ -2721,20 +2791,19 @@ __device__ __forceinline__ void typed_gemm_tile(const GemmArgs& a, uint8_t* lds,
     for (int c = 0; c < CT; ++c)
       asm volatile("" : "+a"(acc[rt][c]));
 
-  const bool full = mt0 * 16 + kG2M <= a.m;
+  float* const elds = reinterpret_cast<float*>(bring);  // this wave's B ring: its loads have landed
   if constexpr (GATED) {
     const int nct2 = ntiles - ct0 >= OT ? OT : ntiles - ct0 > 0 ? ntiles - ct0 : 0;
-    full ? gemm2_epilogue_gated<OutT, true, CT>(a, acc, mt0, ct0, lane, nct2) : gemm2_epilogue_gated<OutT, false, CT>(a, acc, mt0, ct0, lane, nct2);
+    gemm2_epilogue_gated<OutT>(a, acc, mt0, ct0, lane, nct2, elds);
     return;
   }
   const int nct = ntiles - ct0 >= CT ? CT : ntiles - ct0 > 0 ? ntiles - ct0 : 0;
-  float* const lrs = reinterpret_cast<float*>(bring);  // this wave's B ring: its loads have landed
   if (a.post == 0)
-    full ? gemm2_epilogue<OutT, 0, true, CT>(a, acc, mt0, ct0, lane, nct, lrs) : gemm2_epilogue<OutT, 0, false, CT>(a, acc, mt0, ct0, lane, nct, lrs);
+    gemm2_epilogue<OutT, 0>(a, acc, mt0, ct0, lane, nct, elds);
   else if (a.post == 1)
-    full ? gemm2_epilogue<OutT, 1, true, CT>(a, acc, mt0, ct0, lane, nct, lrs) : gemm2_epilogue<OutT, 1, false, CT>(a, acc, mt0, ct0, lane, nct, lrs);
+    gemm2_epilogue<OutT, 1>(a, acc, mt0, ct0, lane, nct, elds);
   else
-    full ? gemm2_epilogue<OutT, 2, true, CT>(a, acc, mt0, ct0, lane, nct, lrs) : gemm2_epilogue<OutT, 2, false, CT>(a, acc, mt0, ct0, lane, nct, lrs);
+    gemm2_epilogue<OutT, 2>(a, acc, mt0, ct0, lane, nct, elds);
 }
 
 // typed_gemm_tile with B in half tile-blocks (policies with kHalf): per
@@ -2923,14 +2992,14 @@ __device__ __forceinline__ void typed_gemm_tile_half(const GemmArgs& a, uint8_t*
     for (int c = 0; c < CT; ++c)
       asm volatile("" : "+a"(acc[rt][c]));
 
-  const bool full = mt0 * 16 + kG2M <= a.m;
+  float* const elds = reinterpret_cast<float*>(bring);  // this wave's half-slots: their loads have landed
   const int nct = ntiles - ct0 >= CT ? CT : ntiles - ct0 > 0 ? ntiles - ct0 : 0;
   if (a.post == 0)
-    full ? gemm2_epilogue<OutT, 0, true, CT>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 0, false, CT>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 0>(a, acc, mt0, ct0, lane, nct, elds);
   else if (a.post == 1)
-    full ? gemm2_epilogue<OutT, 1, true, CT>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 1, false, CT>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 1>(a, acc, mt0, ct0, lane, nct, elds);
   else
-    full ? gemm2_epilogue<OutT, 2, true, CT>(a, acc, mt0, ct0, lane, nct) : gemm2_epilogue<OutT, 2, false, CT>(a, acc, mt0, ct0, lane, nct);
+    gemm2_epilogue<OutT, 2>(a, acc, mt0, ct0, lane, nct, elds);
 }
 
 template <class P>
