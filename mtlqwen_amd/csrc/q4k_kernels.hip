@@ -3514,12 +3514,16 @@ static int split_segments_per_wg(int tiles, int cus) {
 //    segments 0 (b = 27, 30: 119.0, 128.0 us) do not pay for the exchange
 //    they hide.  At K = 4096 the 112-tile O projection measured 56.0 us split
 //    against 50.4 on the template, which it keeps.
-//  - q >= 2 and K >= 4096: b = q nb / (q + 1) rounded up, so that the q
+//  - q = 2 and K >= 4096: b = q nb / (q + 1) rounded up, so that the q
 //    segments 1 of a workgroup take no longer than one segment 0.  The
 //    N = 6144 projection's 168 tiles at M = 821 (b = 11) measured 58.9-60.9
 //    us for b = 10..13 against 64.3 unsplit: the segments 0 run at 5.4 us
 //    per block against 4.0 unsplit, so that 252 workgroups gain only 8 %
 //    over 168.
+//  - q >= 3: no split.  The few free CUs then hold q short segments each, whose
+//    exchanges follow one another: N = 12288 at M = 640 (q = 15) measured 182
+//    us against 77.7 unsplit, its gate/up pair 251 against 139; N = 8192 at
+//    M = 821 (q = 7) 102 against 73.2, at M = 705 (q = 3) 69.1 against 67.9.
 // Returns b, or 0 for no split.  Q4K_GEMM2_SPLIT=0 turns the split off;
 // Q4K_GEMM2_SPLIT_B forces b (for every shape with tiles < CUs and b < nb).
 int gemm2_split_b(int m, int n, int nb, int cus) {
@@ -3533,7 +3537,7 @@ int gemm2_split_b(int m, int n, int nb, int cus) {
   const int q = split_segments_per_wg(tiles, cus);
   if (q == 1)
     return nb >= 32 ? nb / 2 : 0;
-  return nb >= 16 ? (q * nb + q) / (q + 1) : 0;
+  return q == 2 && nb >= 16 ? (q * nb + q) / (q + 1) : 0;
 }
 
 void gemm2_split_workspace(int m, int n, bool gated, size_t* part_floats, size_t* counters) {
