@@ -28,38 +28,31 @@ namespace q4k {
 namespace {
 
 // ----------------------------------------------------------------------------
-// Activation staging.  One workgroup per row.  Rows of up to 256 * 8 * kStageRegChunks
+// Activation staging.  One workgroup of 512 threads per row (K = 4096, 40
+// rows: 3.4 us against 5.3 with 256).  Rows of up to 512 * 8 * kStageRegChunks
 // elements are held in registers between the max reduction and the
 // conversion (one read of x); longer rows are read twice.
 // ----------------------------------------------------------------------------
-constexpr int kStageRegChunks = 6;
+constexpr int kStageThreads = 512, kStageRegChunks = 3;
 
-__device__ __forceinline__ float block_max_256(float mx) {
+// Maximum of mx and sum of ss over the workgroup's threads (one barrier).
+__device__ __forceinline__ void block_max_sum(float& mx, float& ss) {
+  __shared__ float red[2][kStageThreads / 64];
+  mx = max64_lanes(mx);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1)
-    mx = fmaxf(mx, __shfl_xor(mx, off));
-  __shared__ float red[4];
-  if ((threadIdx.x & 63) == 0)
-    red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-
-// Maximum of mx and sum of ss over the 256 threads (one barrier).
-__device__ __forceinline__ void block_max_sum_256(float& mx, float& ss) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    mx = fmaxf(mx, __shfl_xor(mx, off));
     ss += __shfl_xor(ss, off);
-  }
-  __shared__ float red[2][4];
   if ((threadIdx.x & 63) == 0) {
     red[0][threadIdx.x >> 6] = mx;
     red[1][threadIdx.x >> 6] = ss;
   }
   __syncthreads();
-  mx = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-  ss = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+  ss = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kStageThreads / 64; ++w) {
+    mx = fmaxf(mx, red[0][w]);
+    ss += red[1][w];
+  }
 }
 
 // Fused RMS norm of a staged row (native_ops.metal:6-40): the staging
@@ -71,7 +64,7 @@ struct RowNorm {
   float eps = 0.0f;
 };
 
-// Converts and stores one 8-element chunk; all 256 threads of the workgroup
+// Converts and stores one 8-element chunk; all threads of the workgroup
 // must call it together (the sub-block sum is reduced over 4 lanes).
 template <int MODE>
 __device__ __forceinline__ void stage_store(_Float16* xo, _Float16* xs, _Float16* xe, int row, int c, bool live, int m, int k, int nb,
@@ -80,7 +73,11 @@ __device__ __forceinline__ void stage_store(_Float16* xo, _Float16* xs, _Float16
   float sum = 0.0f, res = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const float t = v[i] * up;
+    // One fp32 value for both parts (with a norm `up` is no power of two, and
+    // a product fused into the conversions would be rounded differently in
+    // the stored part and in its residual).
+    float t = v[i] * up;
+    asm("" : "+v"(t));
     hi[i] = (_Float16)t;
     const float r = t - (float)hi[i];
     lo[i] = (_Float16)r;
@@ -133,12 +130,12 @@ __device__ __forceinline__ void load8_norm(const InT* xr, const float* nw, int c
 }
 
 template <typename InT, int MODE, bool NORM>
-__global__ __launch_bounds__(256) void stage_x_kernel(const InT* __restrict__ x, _Float16* __restrict__ xo, _Float16* __restrict__ xs,
+__global__ __launch_bounds__(kStageThreads) void stage_x_kernel(const InT* __restrict__ x, _Float16* __restrict__ xo, _Float16* __restrict__ xs,
                                                       float* __restrict__ rowscale, int m, int k, RowNorm nrm) {
   const int row = blockIdx.x;
   const InT* xr = x + (size_t)row * k;
   const int chunks = k >> 3, nb = k >> 8;
-  const bool in_regs = chunks <= 256 * kStageRegChunks;
+  const bool in_regs = chunks <= kStageThreads * kStageRegChunks;
   // The residual sums' plane follows the sub-block sums (of m rows, or 2m
   // for hi/lo fragments, whose residual sums are written as zeros).
   _Float16* const xe = xs + xs_plane_halves(MODE == kStageFragSplit ? 2 * m : m, nb);
@@ -147,7 +144,7 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const InT* __restrict__ x,
   if (in_regs) {
 #pragma unroll
     for (int j = 0; j < kStageRegChunks; ++j) {
-      const int c = threadIdx.x + 256 * j;
+      const int c = threadIdx.x + kStageThreads * j;
       if (c < chunks) {
         load8_norm<NORM>(xr, nrm.w, c, v[j], ss);
 #pragma unroll
@@ -156,7 +153,7 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const InT* __restrict__ x,
       }
     }
   } else {
-    for (int c = threadIdx.x; c < chunks; c += 256) {
+    for (int c = threadIdx.x; c < chunks; c += kStageThreads) {
       float t[8];
       load8_norm<NORM>(xr, nrm.w, c, t, ss);
 #pragma unroll
@@ -165,12 +162,10 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const InT* __restrict__ x,
     }
   }
   float r = 1.0f;
+  block_max_sum(mx, ss);
   if (NORM) {
-    block_max_sum_256(mx, ss);
     r = 1.0f / sqrtf(ss / (float)k + nrm.eps);
     mx *= r;
-  } else {
-    mx = block_max_256(mx);
   }
   float up, down;
   pow2_scale(mx, up, down);
@@ -180,12 +175,12 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const InT* __restrict__ x,
   if (in_regs) {
 #pragma unroll
     for (int j = 0; j < kStageRegChunks; ++j) {
-      const int c = threadIdx.x + 256 * j;
-      if (256 * j < chunks)  // uniform: whole groups of 4 lanes take part
+      const int c = threadIdx.x + kStageThreads * j;
+      if (kStageThreads * j < chunks)  // uniform: whole groups of 4 lanes take part
         stage_store<MODE>(xo, xs, xe, row, c, c < chunks, m, k, nb, v[j], cs);
     }
   } else {
-    for (int c0 = 0; c0 < chunks; c0 += 256) {
+    for (int c0 = 0; c0 < chunks; c0 += kStageThreads) {
       const int c = c0 + threadIdx.x;
       float t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       float unused = 0.0f;
@@ -3349,15 +3344,15 @@ hipError_t launch_typed_gate_up(hipStream_t s, const GemvArgs& a, uint32_t type,
 
 template <typename InT, bool NORM>
 hipError_t stage_launch(hipStream_t s, const InT* x, _Float16* xo, _Float16* xs, float* rowscale, int m, int k, int mode, RowNorm nrm) {
-  const dim3 grid((unsigned)m), block(256);
+  const dim3 grid((unsigned)m), block(kStageThreads);
   if (mode == kStageFrag)
     (void)dispatch(stage_x_kernel<InT, kStageFrag, NORM>, grid, block, s, x, xo, xs, rowscale, m, k, nrm);
   else if (mode == kStageGemm && k / 256 <= 16)
-    (void)dispatch(stage_gemm_kernel<InT, 16, 32, NORM>, dim3((unsigned)((m + 7) / 8)), block, s, x, xo, rowscale, m, k, nrm);
+    (void)dispatch(stage_gemm_kernel<InT, 16, 32, NORM>, dim3((unsigned)((m + 7) / 8)), dim3(256), s, x, xo, rowscale, m, k, nrm);
   else if (mode == kStageGemm && k % 512 == 0 && k / 512 <= 24)  // K <= 12288: one read of x, 64 threads per row
     (void)dispatch(stage_gemm_kernel<InT, 24, 64, NORM>, dim3((unsigned)((m + 7) / 8)), dim3(512), s, x, xo, rowscale, m, k, nrm);
   else if (mode == kStageGemm)
-    (void)dispatch(stage_gemm_kernel<InT, 0, 32, NORM>, dim3((unsigned)((m + 7) / 8)), block, s, x, xo, rowscale, m, k, nrm);
+    (void)dispatch(stage_gemm_kernel<InT, 0, 32, NORM>, dim3((unsigned)((m + 7) / 8)), dim3(256), s, x, xo, rowscale, m, k, nrm);
   else
     (void)dispatch(stage_x_kernel<InT, kStageFragSplit, NORM>, grid, block, s, x, xo, xs, rowscale, m, k, nrm);
   return hipGetLastError();
