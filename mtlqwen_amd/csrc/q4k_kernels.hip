@@ -2254,6 +2254,62 @@ __global__ __launch_bounds__(256) void embedding_batch_kernel(const uint8_t* __r
 // ----------------------------------------------------------------------------
 constexpr int kNormRegs = 16;
 
+// RMS norm of one row per workgroup of 512 threads, 8 elements (one 16- or
+// two 16-byte loads) per thread and chunk, the row in registers between the
+// sum of squares and the scaling: a single-element form of 16 dependent loads
+// per thread took 11.3 us for 40 fp16 rows of 4096 and 5.9 us for 5.
+constexpr int kNormChunks = 3;
+template <typename T>
+__global__ __launch_bounds__(512) void rms_norm8_kernel(const T* __restrict__ x, const float* __restrict__ w, T* y, int k, float eps, GatherIndex idx,
+                                                        int gather) {
+  const int r = blockIdx.x, tid = threadIdx.x, chunks = k >> 3;
+  const T* xr = x + (size_t)(gather ? idx.src[r] : (uint32_t)r) * k;
+  float v[kNormChunks][8];
+  float ss = 0.0f;
+#pragma unroll
+  for (int j = 0; j < kNormChunks; ++j) {
+    const int c = tid + 512 * j;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      v[j][i] = 0.0f;
+    if (c < chunks)
+      load8(xr + (size_t)c * 8, v[j]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      ss = fmaf(v[j][i], v[j][i], ss);
+  }
+  float nw[kNormChunks][8];
+#pragma unroll
+  for (int j = 0; j < kNormChunks; ++j)
+    if (tid + 512 * j < chunks)
+      load8(w + (size_t)(tid + 512 * j) * 8, nw[j]);
+  __shared__ float part[8];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    ss += __shfl_xor(ss, off);
+  if ((tid & 63) == 0)
+    part[tid >> 6] = ss;
+  __syncthreads();
+  float total = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    total += part[i];
+  const float scale = 1.0f / sqrtf(total / (float)k + eps);
+  T* yr = y + (size_t)r * k;
+#pragma unroll
+  for (int j = 0; j < kNormChunks; ++j) {
+    const int c = tid + 512 * j;
+    if (c < chunks) {
+      typedef T t8 __attribute__((ext_vector_type(8)));
+      t8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        o[i] = (T)((v[j][i] * scale) * nw[j][i]);
+      *reinterpret_cast<t8*>(yr + (size_t)c * 8) = o;
+    }
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const T* __restrict__ x, const float* __restrict__ w, T* y, int k, float eps, GatherIndex idx,
                                                        int gather) {
@@ -3683,18 +3739,29 @@ hipError_t launch_embedding(hipStream_t s, const uint8_t* w, const int32_t* ids,
   return hipGetLastError();
 }
 
+template <typename T>
+static void rms_norm_rows(hipStream_t s, const void* x, const float* w, void* y, int rows, int k, float eps, const GatherIndex& gi, int gather) {
+  const dim3 grid((unsigned)rows);
+  const T* xt = static_cast<const T*>(x);
+  T* yt = static_cast<T*>(y);
+  // Eight elements at a time where rows and addresses allow it.
+  const uintptr_t at = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w);
+  if (k % 8 == 0 && k <= 8 * 512 * kNormChunks && at % 16 == 0)
+    (void)dispatch(rms_norm8_kernel<T>, grid, dim3(512), s, xt, w, yt, k, eps, gi, gather);
+  else
+    (void)dispatch(rms_norm_kernel<T>, grid, dim3(256), s, xt, w, yt, k, eps, gi, gather);
+}
+
 hipError_t launch_rms_norm(hipStream_t s, const void* x, const float* w, void* y, int rows, int k, float eps, int dtype, const GatherIndex* idx) {
   if (rows == 0)
     return hipSuccess;
   GatherIndex gi{};
   if (idx)
     gi = *idx;
-  const dim3 grid((unsigned)rows), block(256);
   if (dtype == kF32)
-    (void)dispatch(rms_norm_kernel<float>, grid, block, s, static_cast<const float*>(x), w, static_cast<float*>(y), k, eps, gi, idx ? 1 : 0);
+    rms_norm_rows<float>(s, x, w, y, rows, k, eps, gi, idx ? 1 : 0);
   else
-    (void)dispatch(rms_norm_kernel<_Float16>, grid, block, s, static_cast<const _Float16*>(x), w, static_cast<_Float16*>(y), k, eps, gi,
-                   idx ? 1 : 0);
+    rms_norm_rows<_Float16>(s, x, w, y, rows, k, eps, gi, idx ? 1 : 0);
   return hipGetLastError();
 }
 
