@@ -1530,9 +1530,9 @@ constexpr int kG2BWave = 2 * 4 * kTileBlockBytes;      // per wave: 2 blocks x 4
 // columns per lane, and the aux of a whole batch of row tiles is loaded, 4
 // columns per lane, before the first of them is stored.  N = 12288, K = 4096,
 // post 1, before and after: fp16 Q8_0 M = 1531 215 -> 184 us, M = 2048 270 ->
-// 231, Q6_K M = 2048 291 -> 249, Q4_K 256 -> 231, IQ4_XS 287 -> 265; fp32 Q8_0
+// 231, Q6_K M = 2048 291 -> 249, Q4_K 256 -> 215, IQ4_XS 287 -> 247; fp32 Q8_0
 // 245 -> 233, Q6_K 263 -> 249 and, with six column tiles, Q4_K at M = 1531 223
-// -> 211, at M = 2048 242 -> 241.
+// -> 200, at M = 2048 242 -> 225.
 constexpr int kEpiLd(int cols) {
   return cols + 4;  // floats per LDS row: the two row halves of a write fall in different banks
 }
@@ -1643,11 +1643,13 @@ __device__ __forceinline__ void gemm2_flush(const GemmArgs& a, float* wl, int mt
   }
 }
 
-// Row tiles whose aux is loaded together: as many as the registers hold (beside
-// six column tiles' accumulators one, and half its columns at a time).
+// Row tiles whose aux is loaded together: as many as the registers hold.  Beside
+// six column tiles' accumulators that is 16 registers, two column tiles of two
+// (fp32) or four row tiles (N = 12288, K = 4096, M = 2048, post 1: Q4_K fp32 224
+// us, fp16 215, against 241 and 231 for one row tile of three columns).
 template <typename OutT, int CT>
 constexpr int epi_batch() {
-  return CT > 4 ? 1 : CT * sizeof(OutT) <= 16 ? 8 : 4;
+  return CT > 4 ? 8 / (int)sizeof(OutT) : CT * sizeof(OutT) <= 16 ? 8 : 4;
 }
 
 template <typename OutT, int POST, int CT>
@@ -1678,7 +1680,7 @@ __device__ __forceinline__ void gemm2_epilogue(const GemmArgs& a, const f4_t (&a
       }
     }
   } else {
-    constexpr int NC = CT > 4 ? CT / 2 : CT;
+    constexpr int NC = CT > 4 ? 2 : CT;
 #pragma unroll
     for (int c0 = 0; c0 < CT; c0 += NC)
       gemm2_flush<OutT, POST, NC, epi_batch<OutT, CT>()>(a, wl, mt0, ct0 + c0, lane, nct - c0, [&](int rt, int c, int v) {
