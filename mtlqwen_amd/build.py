@@ -13,7 +13,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libq4k.so")
-SOURCES = ["q4k_kernels.hip", "q4k_mid.hip", "q4k_rows.hip", "q4k_api.hip", "q4k_gguf.cpp"]
+SOURCES = ["q4k_kernels.hip", "q4k_mid.hip", "q4k_rows.hip", "q4k_decode.hip", "q4k_api.hip", "q4k_gguf.cpp"]
 ARCH = os.environ.get("Q4K_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops: no v_pk_*_f32 in device code (the host pass warns that it

@@ -686,6 +686,30 @@ bool rows_gemm_takes(hipStream_t stream, const Workspace& ws, const q4k_weight* 
   return rows_gemm_fits(stream, ws, m, w->k, s > 1 ? (size_t)s * ((m + 15) / 16 * 16) * w->n * (gated ? 2 : 1) : 0);
 }
 
+// Up to 8 rows with K = 4096, plain or (wu) a gate/up pair of one type: one
+// launch that packs (and normalises) x itself.
+int run_decode_gemv(hipStream_t stream, q4k_weight* w, q4k_weight* wu, const void* x, void* y, const void* aux, uint32_t m, uint32_t post,
+                    uint32_t dtype, const float* norm_w, float eps) {
+  GemvArgs a{};
+  a.w = w->data;
+  a.wu = wu ? wu->data : nullptr;
+  a.x = x;
+  a.y = y;
+  a.aux = aux;
+  a.m = (int)m;
+  a.n = (int)w->n;
+  a.k = (int)w->k;
+  a.nb = (int)(w->k / 256);
+  a.post = (int)post;
+  a.rows = 2 * (int)m;
+  a.split = 1;
+  a.norm_w = norm_w;
+  a.eps = eps;
+  LaunchTimer timer(stream, wu ? Q4K_KERNEL_GEMV_GATED : Q4K_KERNEL_GEMV);
+  Q4K_TRY_HIP(launch_decode_gemv(stream, a, w->type, (int)dtype, device_cus(w->device)), "decode gemv launch");
+  return Q4K_OK;
+}
+
 // Outputs narrower than kGemmMinColumns take the GEMV groups at every row
 // count, as with Q4_K (the per-row bar).
 int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const void* x, void* y, const void* aux, uint32_t m, uint32_t post,
@@ -694,6 +718,8 @@ int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const voi
     return run_typed_gemm_locked(stream, ws, w, x, y, aux, m, post, dtype, norm_w, eps);
   if (rows_gemm_takes(stream, ws, w, m, false))
     return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
+  if (decode_gemv_supported((int)m, (int)(w->k / 256), (int)w->n, false, device_cus(w->device)))
+    return run_decode_gemv(stream, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   int rc = prenorm(stream, ws, w->device, x, norm_w, eps, m, w->k, dtype);
   if (rc)
     return rc;
@@ -726,6 +752,8 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
       return rc;
     return run_gemv_groups_locked(stream, ws, w, x, y, aux, m, post, dtype);
   }
+  if (!wu && decode_gemv_supported((int)m, (int)(w->k / 256), (int)w->n, false, device_cus(w->device)))
+    return run_decode_gemv(stream, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   const bool gemv = kern.kind != kGemm || m <= 16u * kGemvMaxRowTiles;
   const bool split = gemv && gemv_split((int)m);
   const int rows = split ? 2 * (int)m : (int)m;
@@ -767,25 +795,8 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
       return rc;
     return run_gemv_groups_locked(stream, ws, w, x, y, aux, m, post, dtype);
   }
-  if (gemv && wu && gemv_gate_up_supported((int)m, (int)(w->k / 256), (int)w->n)) {
-    // Fused gate/up GEMV: packs x in registers, no staging launch.
-    GemvArgs a{};
-    a.w = w->data;
-    a.wu = wu->data;
-    a.x = x;
-    a.y = y;
-    a.m = (int)m;
-    a.n = (int)w->n;
-    a.k = (int)w->k;
-    a.nb = (int)(w->k / 256);
-    a.rows = 2 * (int)m;
-    a.split = 1;
-    a.norm_w = norm_w;
-    a.eps = eps;
-    LaunchTimer timer(stream, Q4K_KERNEL_GEMV_GATED);
-    Q4K_TRY_HIP(launch_gemv_gate_up(stream, a, (int)dtype, device_cus(w->device)), "gemv gate/up launch");
-    return Q4K_OK;
-  }
+  if (gemv && wu && decode_gemv_supported((int)m, (int)(w->k / 256), (int)w->n, true, device_cus(w->device)))
+    return run_decode_gemv(stream, w, wu, x, y, nullptr, m, post, dtype, norm_w, eps);
   if (gemv && !wu && q4k_persistent_supported((int)m, (int)(w->k / 256), (int)w->n, device_cus(w->device))) {
     // Wide plain projections (the LM head): the persistent GEMV, x fragments
     // resident in registers.
@@ -1277,29 +1288,15 @@ int mlp_gate_up_impl(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x
     return fail(Q4K_ESHAPE, "decode batch of %u rows exceeds %d", m, 16 * kGemvMaxRowTiles);
   if (phase == Q4K_PHASE_GATED_DECODE && q4)
     return run_linear(s, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, phase, norm_w, eps);
-  if (phase == Q4K_PHASE_GATED_DECODE && wg->type == wu->type && typed_gate_up_supported(wg->type, (int)m, (int)(wg->k / 256), (int)wg->n)) {
-    // The fused gate/up GEMV of a type with one in the reference
-    // (fused_kernels.metal:80-200): one launch, x packed in registers.
+  if (phase == Q4K_PHASE_GATED_DECODE && wg->type == wu->type &&
+      decode_gemv_supported((int)m, (int)(wg->k / 256), (int)wg->n, true, device_cus(wg->device))) {
+    // Pairs of another type (fused in the reference for Q5_K and IQ4_XS,
+    // fused_kernels.metal:80-200).
     Workspace& ws = workspace(wg->device);
     std::lock_guard<std::mutex> lock(ws.mu);
     resolve(wg, phase);
     resolve(wu, phase);
-    GemvArgs a{};
-    a.w = wg->data;
-    a.wu = wu->data;
-    a.x = x;
-    a.y = y;
-    a.m = (int)m;
-    a.n = (int)wg->n;
-    a.k = (int)wg->k;
-    a.nb = (int)(wg->k / 256);
-    a.rows = 2 * (int)m;
-    a.split = 1;
-    a.norm_w = norm_w;
-    a.eps = eps;
-    LaunchTimer timer(s, Q4K_KERNEL_GEMV_GATED);
-    Q4K_TRY_HIP(launch_typed_gate_up(s, a, wg->type, (int)dtype, device_cus(wg->device)), "typed gate/up launch");
-    return Q4K_OK;
+    return run_decode_gemv(s, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, norm_w, eps);
   }
   Workspace& ws = workspace(wg->device);
   std::lock_guard<std::mutex> lock(ws.mu);

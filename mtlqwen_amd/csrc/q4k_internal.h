@@ -425,10 +425,6 @@ struct GemvShape {
 // column tiles and waves per workgroup, for tuning.
 GemvShape gemv_shape(int rows, int n, int nb, bool gated, int cus);
 
-// Fused gate/up GEMV for m <= 8 rows and K = 4096 that packs x itself (no
-// staging launch); reads a.x, a.w, a.wu (and a.norm_w when set) and writes a.y.
-bool gemv_gate_up_supported(int m, int nb, int n);
-hipError_t launch_gemv_gate_up(hipStream_t s, const GemvArgs& a, int dtype, int cus);
 // GEMV over staged x of 17..48 fragment rows: T column tiles of NM matrices
 // per workgroup, 8 waves splitting K (K = 2048 .. 12288), each block of x
 // read once per wave.  gemv_rows_plan returns T (0: not this kernel) and the
@@ -440,10 +436,11 @@ struct RowsPlan {
 RowsPlan gemv_rows_plan(int rows, int nb, int n, bool gated, int cus);
 size_t gemv_rows_part_floats(const RowsPlan& p, int n);
 hipError_t launch_gemv_rows(hipStream_t s, const GemvArgs& a, int dtype, const RowsPlan& p, bool gated);
-// The same for gate and up weights of one other type with a fused decode
-// kernel in the reference (Q5_K, IQ4_XS).
-bool typed_gate_up_supported(uint32_t type, int m, int nb, int n);
-hipError_t launch_typed_gate_up(hipStream_t s, const GemvArgs& a, uint32_t type, int dtype, int cus);
+// One-launch decode GEMV, m <= 8 rows and K = 4096, every weight type
+// (q4k_decode.hip): reads a.x (normalised with a.norm_w when set), a.w and
+// a.aux, or a.w and a.wu for a gate/up pair; packs x itself (no staging launch).
+bool decode_gemv_supported(int m, int nb, int n, bool gated, int cus);
+hipError_t launch_decode_gemv(hipStream_t s, const GemvArgs& a, uint32_t type, int dtype, int cus);
 
 // Split-K GEMV for m <= 8 (see q4k_gemv_splitk_kernel): a plan picks an
 // instance for (n, nb); the launch needs `part` (gemv_splitk_part_floats

@@ -4,9 +4,8 @@
 //  stage_x_kernel, stage_gemm_kernel, stage_pack_kernel
 //                   activations -> fp16 operands with power-of-two scales
 //  q4k_gemv_kernel  staged decode GEMV (up to 48 rows), optionally gated
-//  q4k_gemv_gate_up_kernel   fused gate/up decode GEMV, x packed in registers
 //  q4k_gemv_splitk_kernel    split-K decode GEMV (K = 12288)
-//  typed_gemv_kernel, typed_gemv_persistent_kernel, typed_gate_up_kernel
+//  typed_gemv_kernel, typed_gemv_persistent_kernel
 //                   decode GEMVs over a format policy (Q6_K, Q8_0, Q5_K,
 //                   IQ4_XS; Q4_K for the wide LM head)
 //  q4k_gemm2_kernel, typed_gemm_kernel
@@ -22,7 +21,7 @@
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
 
-#include "q4k_formats.h"
+#include "q4k_pack.h"
 
 namespace q4k {
 namespace {
@@ -590,380 +589,6 @@ __global__ __launch_bounds__(64 * W) void q4k_gemv_kernel(GemvArgs a) {
 // ----------------------------------------------------------------------------
 // Load helpers of the GEMVs that stream weights through LDS.
 // ----------------------------------------------------------------------------
-
-// ----------------------------------------------------------------------------
-// Fused gate/up GEMV with in-register activation packing (m <= 8 rows, K =
-// 4096, N = 16 T x workgroups: one item of T column tiles per workgroup).
-//
-// Wave w owns K-blocks bw, bw + 1 (bw = 2 ((w + b) % 8), rotated so that the
-// workgroups of one L2 read different parts of x first) of the workgroup's T
-// column tiles of both matrices: U = 4T tile-blocks ("units").  It loads its
-// two blocks of x (one coalesced 1 KB load per (block, row)), then keeps two
-// units in flight ahead of the pair it computes (per unit the 16-byte header
-// row of the lane's column and the two quant slabs, 16 B per lane).  No
-// staging launch precedes it: while
-// the first units are in flight the wave turns its blocks of x into the MFMA
-// operands in registers, with the same arithmetic as the decode pack
-// (pack_block_row):
-//  - x passes through LDS so that lane 16g + i holds elements
-//    64g + 32 (i / 8) + [0, 32) of row i % 8 (rows >= m read as zero);
-//  - each (row, block) is scaled by a power of two that puts its largest
-//    magnitude in [2^14, 2^15) and split into hi = h(t), lo = h(t - hi);
-//  - lanes i and i ^ 8 (one DPP row rotation) trade halves so that lanes
-//    i < 8 hold the high parts of elements 64g + [0, 64) of row i and lanes
-//    i >= 8 the low parts: the A fragments of v_mfma_f32_16x16x32_f16, rows
-//    8..15 carrying the low parts;
-//  - each lane's 32 elements are one sub-block; their sums / 32 (hi / lo)
-//    are gathered into the min-term operand of v_mfma_f32_16x16x16_f16.
-// Units are computed two at a time, their instruction streams interleaved.
-// The partial sums of a unit are unscaled and accumulated in registers; hi
-// and lo rows are combined (lanes l, l + 32) and the eight waves' sums are
-// added in wave order through LDS before the SiLU(gate) * up epilogue.  The
-// kernel is bound by its vector ALU: about 135 VALU instructions per unit
-// and 500 for the pack, two waves per SIMD.
-// ----------------------------------------------------------------------------
-constexpr int kDppRowRor8 = 0x128;  // lane i <- lane (i + 8) % 16 within 16 lanes
-
-template <int BANKS>
-__device__ __forceinline__ uint32_t ror8_into(uint32_t old, uint32_t src) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kDppRowRor8, 0xF, BANKS, false);
-}
-
-// Registers of one packed x block: A fragments, min-term operand and the
-// unscale factors of this lane's C rows (4g + v) & 7.
-struct XBlock {
-  h8_t frag[8];
-  h4_t xs;
-  float dv[4];
-};
-
-// Converts the 32 values t0 (elements 64g + 32 (i / 8) + [0, 32) of row i % 8,
-// lane 16g + i) of one block into the block's operands.
-__device__ __forceinline__ void pack_x_regs(const float (&xv)[32], int lane, XBlock& xb) {
-  const int g = lane >> 4, i = lane & 15, half = i >> 3;
-  // Largest magnitude of the (row, block): own 32, the partner half, the four
-  // lane groups.
-  float mx = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 32; ++e)
-    mx = fmaxf(mx, fabsf(xv[e]));
-  mx = fmaxf(mx, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, mx), kDppRowRor8, 0xF, 0xF, false)));
-  mx = fmaxf(mx, __shfl_xor(mx, 16));
-  mx = fmaxf(mx, __shfl_xor(mx, 32));
-  float up = 1.0f, down = 1.0f;
-  if (mx > 0.0f && mx <= FLT_MAX) {
-    int ex;
-    frexpf(mx, &ex);
-    ex = ex < -80 ? -80 : ex;
-    up = ldexpf(1.0f, 15 - ex);
-    down = ldexpf(1.0f, ex - 15);
-  }
-  uint32_t hw[16], lw[16];
-  float sum = 0.0f;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const float t0 = xv[2 * v] * up, t1 = xv[2 * v + 1] * up;
-    sum += t0 + t1;
-    const h2_t h = __builtin_bit_cast(h2_t, __builtin_amdgcn_cvt_pkrtz(t0, t1));
-    hw[v] = __builtin_bit_cast(uint32_t, h);
-    lw[v] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(t0 - (float)h[0], t1 - (float)h[1]));
-  }
-  // Fragments 0..3 (elements 64g + [0, 32)): own high parts in lanes i < 8,
-  // the partner's low parts in lanes i >= 8 (banks 2, 3 take the rotation).
-  // Fragments 4..7 (64g + [32, 64)): the partner's high parts in lanes i < 8,
-  // own low parts in lanes i >= 8.
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    u4_t f0, f1;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      f0[v] = ror8_into<0xC>(hw[4 * s + v], lw[4 * s + v]);
-      f1[v] = ror8_into<0x3>(lw[4 * s + v], hw[4 * s + v]);
-    }
-    xb.frag[s] = __builtin_bit_cast(h8_t, f0);
-    xb.frag[4 + s] = __builtin_bit_cast(h8_t, f1);
-  }
-  // Sub-block sums / 32 as (hi, lo) halves; lane 16G + r (G < 2) gathers
-  // sub-blocks 4G + c (c = 0..3) of row r % 8 from lanes 16 (2G + c / 2) +
-  // r % 8 + 8 (c % 2), taking the high halves for r < 8 and the low for r >= 8.
-  const float s32 = sum * 0.03125f;
-  const _Float16 sh = (_Float16)s32;
-  const _Float16 sl = (_Float16)(s32 - (float)sh);
-  const uint32_t shl = (uint32_t)__builtin_bit_cast(uint16_t, sh) | ((uint32_t)__builtin_bit_cast(uint16_t, sl) << 16);
-  const int G = g & 1, r8 = i & 7;
-  uint32_t got[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-    got[c] = (uint32_t)__shfl((int)shl, 16 * (2 * G + (c >> 1)) + r8 + 8 * (c & 1));
-  const uint32_t sel = half ? 0x07060302u : 0x05040100u;  // low or high halves of a pair of dwords
-  const uint32_t x01 = __builtin_amdgcn_perm(got[1], got[0], sel), x23 = __builtin_amdgcn_perm(got[3], got[2], sel);
-  xb.xs = g < 2 ? __builtin_bit_cast(h4_t, uint2{x01, x23}) : h4_t{(_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f, (_Float16)0.0f};
-  // Unscale factors of C rows 4 (g & 1) + v (the same in every lane of a row).
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const float d0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, down), v));
-    const float d1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, down), 4 + v));
-    xb.dv[v] = (g & 1) ? d1 : d0;
-  }
-}
-
-// x of wave w, re-ordered for the register pack: [block][lane][32 + 4]
-// floats (the 4-float pad makes the 16-byte reads of 16 lanes hit 64
-// distinct banks), BPW blocks per wave.  The partial sums reuse the wave's
-// own region at the end.
-constexpr int kGuXRow = 36;
-template <int BPW>
-constexpr int gu_wave_floats() {
-  return BPW * 64 * kGuXRow;
-}
-
-// The x of one item of the fused gate/up GEMV, packed: wave w loads K-blocks
-// bw, bw + 1 of all 8 rows (one coalesced load per (block, row), lane l
-// holding elements 4l..4l+3; rows >= m read row 0 and are zeroed), calls
-// issue_first() once its x has landed, and turns its blocks into MFMA
-// operands in registers (through its LDS region).  NORM: x
-// is RMS-normalised on the way in (native_ops.metal:6-40, the norm
-// forward.cpp:114 applies before the MLP): the 8 waves hold all of x between
-// them, so each row's sum of squares is their partial sums (ssq [wave][row])
-// added after one barrier, and every element becomes
-// (x * rsqrt(sum / k + eps)) * w before the pack.
-template <typename OutT, bool NORM, int W, int BPW, typename Issue>
-__device__ __forceinline__ void gate_up_pack_x(const GemvArgs& a, float* xl, float (*ssq)[8], int bw, XBlock (&xb)[BPW],
-                                               Issue&& issue_first) {
-  constexpr int kXRow = kGuXRow;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  float xv[BPW][8][4];
-#pragma unroll
-  for (int j = 0; j < BPW; ++j)
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const OutT* p = reinterpret_cast<const OutT*>(a.x) + (size_t)(r < a.m ? r : 0) * a.k + (size_t)(bw + j) * 256 + 4 * lane;
-      if (sizeof(OutT) == 4) {
-        const f4_t v4 = *reinterpret_cast<const f4_t*>(p);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          xv[j][r][e] = v4[e];
-      } else {
-        const h4_t v4 = *reinterpret_cast<const h4_t*>(p);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          xv[j][r][e] = (float)v4[e];
-      }
-    }
-  f4_t nw[BPW];
-  if constexpr (NORM) {
-#pragma unroll
-    for (int j = 0; j < BPW; ++j)
-      nw[j] = *reinterpret_cast<const f4_t*>(a.norm_w + (size_t)(bw + j) * 256 + 4 * lane);
-  }
-  __builtin_amdgcn_sched_barrier(0);
-
-  if constexpr (NORM) {
-    float ss[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      ss[r] = 0.0f;
-#pragma unroll
-      for (int j = 0; j < BPW; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          ss[r] = fmaf(xv[j][r][e], xv[j][r][e], ss[r]);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1)
-        ss[r] += __shfl_xor(ss[r], off);
-    }
-    if (lane < 8) {
-      float v = ss[0];
-#pragma unroll
-      for (int r = 1; r < 8; ++r)
-        v = lane == r ? ss[r] : v;
-      ssq[wave][lane] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      float tot = 0.0f;
-#pragma unroll
-      for (int w = 0; w < W; ++w)
-        tot += ssq[w][r];
-      const float scale = 1.0f / sqrtf(tot / (float)a.k + a.eps);
-#pragma unroll
-      for (int j = 0; j < BPW; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          xv[j][r][e] = (xv[j][r][e] * scale) * nw[j][e];
-    }
-  }
-  // Element e = 4 lane of row r goes to pack lane 16 (e / 64) + r + 8 ((e / 32) & 1),
-  // float (e & 31) of its 32.
-  float* const xw = xl + (size_t)wave * gu_wave_floats<BPW>();
-  const int dl = 16 * (lane >> 4) + 8 * ((lane >> 3) & 1), doff = 4 * (lane & 7);
-#pragma unroll
-  for (int j = 0; j < BPW; ++j)
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      f4_t v4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v4[e] = r < a.m ? xv[j][r][e] : 0.0f;
-      *reinterpret_cast<f4_t*>(xw + (j * 64 + dl + r) * kXRow + doff) = v4;
-    }
-  // The first weight loads go out once x has landed, not with it: issued
-  // together, every wave's first units queue ahead of the x of later
-  // workgroups (measured: kernel 15.0 against 15.6 us at config 1).  The
-  // LDS transposition and the register pack below run under them.
-  __builtin_amdgcn_sched_barrier(0);
-  issue_first();
-  __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int j = 0; j < BPW; ++j) {
-    float t32[32];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const f4_t v4 = *reinterpret_cast<const f4_t*>(xw + (j * 64 + lane) * kXRow + 4 * c);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        t32[4 * c + e] = v4[e];
-    }
-    pack_x_regs(t32, lane, xb[j]);
-  }
-}
-
-// The end of an item: C row 4g + v of each (matrix, tile) pair, lanes g < 2
-// adding the low part held 32 lanes up, goes to the wave's LDS region; the
-// eight waves' sums are added in wave order and SiLU(gate) * up is stored.
-template <int T, typename OutT, int W, int BPW>
-__device__ __forceinline__ void gate_up_finish(const GemvArgs& a, float* xl, const f4_t (&acc)[2 * T], int item) {
-  constexpr int MT = 2 * T, WF = gu_wave_floats<BPW>();
-  static_assert(MT * 8 * 16 <= WF, "partials fit the x region");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, col = lane & 15;
-  float* const xw = xl + (size_t)wave * WF;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float tot = acc[mt][v] + __shfl_xor(acc[mt][v], 32);
-      if (g < 2)
-        xw[(mt * 8 + 4 * g + v) * 16 + col] = tot;
-    }
-  __syncthreads();
-  OutT* y = reinterpret_cast<OutT*>(a.y);
-  constexpr int EPI = 16 * T;
-  for (int o = tid; o < a.m * EPI; o += 64 * W) {
-    const int row = o / EPI, c = o % EPI, t = c >> 4, cc = c & 15;
-    float gv = 0.0f, uv = 0.0f;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      gv += xl[w * WF + (t * 8 + row) * 16 + cc];
-      uv += xl[w * WF + ((T + t) * 8 + row) * 16 + cc];
-    }
-    if (sizeof(OutT) == 2) {
-      gv = round_half(gv);
-      uv = round_half(uv);
-    }
-    store_elem(y, (size_t)row * a.n + ((size_t)item * T + t) * 16 + cc, silu(gv) * uv);
-  }
-}
-
-// One item (T column tiles of both matrices) of the fused gate/up GEMV, by the
-// 8 waves of the workgroup.
-template <int T, typename OutT, bool NORM, int W, int BPW>
-__device__ __forceinline__ void gate_up_item(const GemvArgs& a, float* xl, float (*ssq)[8], int item) {
-  constexpr int NM = 2, MT = NM * T, U = BPW * MT;
-  static_assert(W * BPW == 16, "the waves cover the 16 blocks of K = 4096");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, col = lane & 15;
-  const int nb = a.nb, bw = ((wave + item) % W) * BPW;
-  const size_t tile_bytes = (size_t)nb * kTileBlockBytes;
-
-  // Units are loaded into registers DQ ahead of the one being computed
-  // (header dword, then the two quant slabs; the scheduling barriers keep
-  // the issue order: x first, then unit by unit, the first units once x has
-  // landed).  A shallow window keeps the memory queues short, so x and each
-  // wave's next unit arrive early; issuing more units ahead measured slower
-  // (they queue ahead of the x of later workgroups).
-  // Units are loaded into registers two ahead of the pair being computed:
-  // the header row of the lane's own column (16 bytes; four lanes share
-  // one row), then the two quant slabs.  The scheduling barriers keep the
-  // issue order: x first, then unit by unit, the first units once x has
-  // landed.  A shallow window keeps the memory queues short, so x and each
-  // wave's next units arrive early (deeper windows measured no faster).
-  constexpr int DQ = 2;
-  static_assert(U % 2 == 0 && MT % 2 == 0, "pairs of units within one block");
-  u4_t hdr[U], q0[U], q1[U];
-  auto issue_unit = [&](int u) {
-    const int j = u / MT, mt = u - j * MT, mi = mt / T, t = mt - mi * T;
-    const uint8_t* src = (mi ? a.wu : a.w) + ((size_t)item * T + t) * tile_bytes + (size_t)(bw + j) * kTileBlockBytes;
-    hdr[u] = __builtin_nontemporal_load(reinterpret_cast<const u4_t*>(src + kHeaderOffset) + col);
-    q0[u] = __builtin_nontemporal_load(reinterpret_cast<const u4_t*>(src) + lane);
-    q1[u] = __builtin_nontemporal_load(reinterpret_cast<const u4_t*>(src + kSlabBytes) + lane);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  XBlock xb[BPW];
-  gate_up_pack_x<OutT, NORM, W, BPW>(a, xl, ssq, bw, xb, [&] {
-#pragma unroll
-    for (int u = 0; u < (DQ < U ? DQ : U); ++u)
-      issue_unit(u);
-  });
-
-  f4_t acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-    acc[mt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  // Two units per step, their instruction streams interleaved: the block
-  // constants, nibble decode, MFMA chains and accumulator updates of two
-  // independent tile-blocks of one K-block.  Units 2p + 2, 2p + 3 are
-  // loaded during step p.
-#pragma unroll
-  for (int p = 0; p < U / 2; ++p) {
-    const int u0 = 2 * p, j = u0 / MT, mt0 = u0 - j * MT;
-    __builtin_amdgcn_sched_barrier(0);
-    if (u0 + DQ < U) {
-      issue_unit(u0 + 2);
-      issue_unit(u0 + 3);
-    }
-    BlockConsts kc[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-      kc[e] = block_consts(hdr[u0 + e], g);
-    f4_t cl[2], ch[2], cm[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-      cl[e] = ch[e] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const u4_t qq = s < 2 ? q0[u0 + e] : q1[u0 + e];
-        const uint32_t wa = qq[2 * (s & 1)], wb = qq[2 * (s & 1) + 1];
-        const h8_t blo = quant_times_scale(wa, wb, 0x000F000Fu, 0x64006400u, kc[e].mul_lo, kc[e].add_lo);
-        const h8_t bhi = quant_times_scale(wa, wb, 0x00F000F0u, 0x64006400u, kc[e].mul_hi, kc[e].add_hi);
-        cl[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[j].frag[s], blo, cl[e], 0, 0, 0);
-        ch[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xb[j].frag[4 + s], bhi, ch[e], 0, 0, 0);
-      }
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-      cm[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(xb[j].xs, kc[e].bmin, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-    for (int e = 0; e < 2; ++e)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        acc[mt0 + e][v] += fmaf(kc[e].d, cl[e][v] + ch[e][v], -kc[e].dmin * cm[e][v]) * xb[j].dv[v];
-  }
-  gate_up_finish<T, OutT, W, BPW>(a, xl, acc, item);
-}
-
-template <int T, typename OutT, bool NORM, int W>
-__global__ __launch_bounds__(64 * W) void q4k_gemv_gate_up_kernel(GemvArgs a) {
-  constexpr int BPW = 16 / W;
-  __shared__ __attribute__((aligned(16))) float xl[W * gu_wave_floats<BPW>()];
-  __shared__ float ssq[W][8];
-  gate_up_item<T, OutT, NORM, W, BPW>(a, xl, ssq, blockIdx.x);
-}
 
 // ----------------------------------------------------------------------------
 // GEMV for staged activations of 17..48 fragment rows (the decode pass of a
@@ -2436,62 +2061,6 @@ __device__ __forceinline__ void typed_epilogue(const GemvArgs& a, const float* p
   }
 }
 
-// Fused gate/up GEMV of a weight type with a fused decode kernel in the
-// reference (Q5_K, IQ4_XS: fused_kernels.metal:80-143, 145-200): the Q4_K
-// item's x packing and epilogue (gate_up_pack_x, gate_up_finish) around the
-// type's tile-block units (F::load, F::mac), two units in flight per wave.
-template <class F, int T, typename OutT, bool NORM>
-__device__ __forceinline__ void typed_gate_up_item(const GemvArgs& a, float* xl, float (*ssq)[8], int item) {
-  constexpr int W = 8, BPW = 2, NM = 2, MT = NM * T, U = BPW * MT, DQ = 2;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nb = a.nb, bw = ((wave + item) % W) * BPW;
-  const size_t tile_bytes = (size_t)nb * F::kTB;
-  typename F::U un[U];
-  auto issue_unit = [&](int u) {
-    const int j = u / MT, mt = u - j * MT, mi = mt / T, t = mt - mi * T;
-    F::load(un[u], (mi ? a.wu : a.w) + ((size_t)item * T + t) * tile_bytes + (size_t)(bw + j) * F::kTB, lane);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  XBlock xb[BPW];
-  gate_up_pack_x<OutT, NORM, W, BPW>(a, xl, ssq, bw, xb, [&] {
-#pragma unroll
-    for (int u = 0; u < (DQ < U ? DQ : U); ++u)
-      issue_unit(u);
-  });
-  XF xf[BPW];
-#pragma unroll
-  for (int j = 0; j < BPW; ++j) {
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-      xf[j].f[s] = xb[j].frag[s];
-    xf[j].xs = xb[j].xs;
-#pragma unroll
-    for (int v = 0; v < 4; ++v)
-      xf[j].dv[v] = xb[j].dv[v];
-  }
-  f4_t acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-    acc[mt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int j = u / MT, mt = u - j * MT;
-    __builtin_amdgcn_sched_barrier(0);
-    if (u + DQ < U)
-      issue_unit(u + DQ);
-    F::mac(un[u], xf[j], lane, acc[mt]);
-  }
-  gate_up_finish<T, OutT, W, BPW>(a, xl, acc, item);
-}
-
-template <class F, int T, typename OutT, bool NORM>
-__global__ __launch_bounds__(512) void typed_gate_up_kernel(GemvArgs a) {
-  __shared__ __attribute__((aligned(16))) float xl[8 * gu_wave_floats<2>()];
-  __shared__ float ssq[8][8];
-  typed_gate_up_item<F, T, OutT, NORM>(a, xl, ssq, blockIdx.x);
-}
-
 template <class F, int T, int DQ, typename OutT>
 __global__ __launch_bounds__(512) void typed_gemv_kernel(GemvArgs a) {
   constexpr int W = 8;
@@ -3330,73 +2899,6 @@ hipError_t launch_gemv_rows(hipStream_t s, const GemvArgs& a, int dtype, const R
     case 2: return gemv_rows_rt<1, 2>(s, a, dtype);
     case 1: return gemv_rows_rt<1, 1>(s, a, dtype);
     default: return hipErrorInvalidValue;
-  }
-}
-
-bool gemv_gate_up_supported(int m, int nb, int n) {
-  static const bool enabled = env_int("Q4K_GEMV_GATE_UP", 1) != 0;
-  return enabled && m >= 1 && m <= 8 && nb == 16 && n % 16 == 0;
-}
-
-// Eight waves per workgroup, two K-blocks each.  (Sixteen waves of one
-// block each need more than their 128 registers and spill.)
-constexpr int kGuWaves = 8;
-
-template <int T, bool NORM>
-hipError_t gate_up_launch(hipStream_t s, const GemvArgs& a, int dtype, unsigned grid) {
-  if (dtype == kF32)
-    (void)dispatch(q4k_gemv_gate_up_kernel<T, float, NORM, kGuWaves>, dim3(grid), dim3(64 * kGuWaves), s, a);
-  else
-    (void)dispatch(q4k_gemv_gate_up_kernel<T, _Float16, NORM, kGuWaves>, dim3(grid), dim3(64 * kGuWaves), s, a);
-  return hipGetLastError();
-}
-
-hipError_t launch_gemv_gate_up(hipStream_t s, const GemvArgs& a, int dtype, int cus) {
-  // Three column tiles per workgroup while that still gives every CU one
-  // workgroup (N = 12288: 256); otherwise one.
-  const int ctiles = a.n / 16;
-  const bool t3 = ctiles % 3 == 0 && ctiles / 3 >= cus;
-  const unsigned grid = (unsigned)(t3 ? ctiles / 3 : ctiles);
-  if (a.norm_w)
-    return t3 ? gate_up_launch<3, true>(s, a, dtype, grid) : gate_up_launch<1, true>(s, a, dtype, grid);
-  return t3 ? gate_up_launch<3, false>(s, a, dtype, grid) : gate_up_launch<1, false>(s, a, dtype, grid);
-}
-
-bool typed_gate_up_supported(uint32_t type, int m, int nb, int n) {
-  static const bool enabled = env_int("Q4K_GEMV_GATE_UP", 1) != 0;
-  return enabled && (type == kTypeQ5_K || type == kTypeIQ4_XS) && m >= 1 && m <= 8 && nb == 16 && n % 16 == 0;
-}
-
-template <class F, int T, bool NORM>
-hipError_t typed_gate_up_launch(hipStream_t s, const GemvArgs& a, int dtype, unsigned grid) {
-  if (dtype == kF32)
-    (void)dispatch(typed_gate_up_kernel<F, T, float, NORM>, dim3(grid), dim3(512), s, a);
-  else
-    (void)dispatch(typed_gate_up_kernel<F, T, _Float16, NORM>, dim3(grid), dim3(512), s, a);
-  return hipGetLastError();
-}
-
-template <class F>
-hipError_t typed_gate_up_dispatch(hipStream_t s, const GemvArgs& a, int dtype, int cus) {
-  // Column tiles per workgroup as for Q4_K.
-  const int ctiles = a.n / 16;
-  const bool t3 = ctiles % 3 == 0 && ctiles / 3 >= cus;
-  const unsigned grid = (unsigned)(t3 ? ctiles / 3 : ctiles);
-  if (a.norm_w)
-    return t3 ? typed_gate_up_launch<F, 3, true>(s, a, dtype, grid) : typed_gate_up_launch<F, 1, true>(s, a, dtype, grid);
-  return t3 ? typed_gate_up_launch<F, 3, false>(s, a, dtype, grid) : typed_gate_up_launch<F, 1, false>(s, a, dtype, grid);
-}
-
-hipError_t launch_typed_gate_up(hipStream_t s, const GemvArgs& a, uint32_t type, int dtype, int cus) {
-  if (a.m < 1 || a.m > 8 || a.nb != 16 || a.n % 16 != 0)
-    return hipErrorInvalidValue;
-  switch (type) {
-    case kTypeQ5_K:
-      return typed_gate_up_dispatch<FmtQ5K>(s, a, dtype, cus);
-    case kTypeIQ4_XS:
-      return typed_gate_up_dispatch<FmtIQ4XS>(s, a, dtype, cus);
-    default:
-      return hipErrorInvalidValue;
   }
 }
 
