@@ -151,7 +151,8 @@ int q4k_linear_noalloc(void* stream, q4k_weight* w, const void* x, void* y, cons
                        uint32_t nqueries, uint32_t post, uint32_t dtype);
 
 /* Gated MLP projection (model/qwen35/forward.cpp:115-118).
- * Decode passes: one fused gate/up kernel, y = silu(x.Wg^T) * (x.Wu^T)
+ * Decode passes, and short prefill passes whose pair has a fused kernel for
+ * their row count: one fused gate/up kernel, y = silu(x.Wg^T) * (x.Wu^T)
  * (fused_kernels.metal:44-78).  Other passes: the result of the reference's
  * two calls, gate with post 0 into y, then up with post 2 over y in place;
  * Q4_K pairs at prefill row counts compute it in one gated GEMM launch (y
