@@ -14,36 +14,40 @@ namespace {
 
 
 // ---- the kernel --------------------------------------------------------------
-// y = post(x W^T) for row blocks of 16 RT rows.  Workgroup = 8 waves = KG
-// K-groups x 8 / KG column groups of CT column tiles; it takes one row block,
-// one column block and one K-slice (blocks [kb0, kb0 + nbr)).  A step is half
-// a block, u-steps 2h and 2h + 1: with KG = 2 the waves of K-group kg take
-// u-step 2h + kg, with KG = 1 every wave takes both.  The activations of a
+// y = post(x W^T) for row blocks of 16 RT rows.  Workgroup = 8 waves = 2
+// K-groups x 4 column groups of CT column tiles; it takes one row block, one
+// column block and one K-slice (blocks [kb0, kb0 + nbr)).  A step is half a
+// block, u-steps 2h and 2h + 1, of which the waves of K-group kg take 2h + kg.  The activations of a
 // step (RT x 4 KB) arrive by LDS-DMA in a ring of NS slots, NS - 1 steps
 // ahead, the tile-blocks of a block in a ring of NB slots; each tile-block is
 // dequantised once per K-group, into registers, and multiplied into all RT
 // row tiles.
-template <class P, int RT, int CT, int KG, int NS, int NB>
+template <class P, int RT, int CT, int NS, int NB>
 struct MidShape {
-  static constexpr int kCG = 8 / KG, kTiles = kCG * CT, kASlot = RT * 4096, kBSlot = kTiles * P::kTB;
-  static constexpr int kLds = NS * kASlot + NB * kBSlot, kHR = KG == 2 ? RT / 2 : RT;
+  static constexpr int kCG = 4, kTiles = kCG * CT, kASlot = RT * 4096, kBSlot = kTiles * P::kTB;
+  static constexpr int kLds = NS * kASlot + NB * kBSlot, kHR = RT / 2;
   static_assert(kLds <= 160 * 1024, "LDS of one workgroup");
-  static_assert(KG == 1 || 8 * (RT / 2) * CT * 1024 <= kLds, "K-group exchange");
+  static_assert(8 * (RT / 2) * CT * 1024 <= kLds, "K-group exchange");
 };
 
 // The steps of one wave of K-group KGI (compile-time, so that the u-steps and
 // with them the dequantisation's shifts are).
-template <class P, int RT, int CT, int KG, int NS, int NB, bool GATED, int KGI>
+template <class P, int RT, int CT, int NS, int NB, bool GATED, int KGI>
 __device__ __forceinline__ void mid_steps(const MidArgs& a, uint8_t* lds, int by, int cb, int kb0, int nbr, int wave, int lane, f4_t (&acc)[RT][CT]) {
-  using M = MidShape<P, RT, CT, KG, NS, NB>;
-  constexpr int OT = GATED ? CT / 2 : CT, AD = NS - 1, NU = 2 / KG;
+  using M = MidShape<P, RT, CT, NS, NB>;
+  // With four row tiles a step's loads are issued after its first MFMAs, which
+  // need nothing but what the previous step read (gate/up 4096 -> 12288 at 64
+  // rows 34.6 -> 30.7 us, down 26.3 -> 24.6); with eight, where the MFMAs of a
+  // step cover them, before (the late issue took 1 to 3 % more).
+  constexpr bool kLate = RT == 4;
+  constexpr int OT = GATED ? CT / 2 : CT, AD = NS - 1;
   // Tile-blocks this wave loads per block: its columns', shared out between
-  // the two waves that use them (KG = 2; one column: by the first).
-  constexpr int MB = KG == 1 ? CT : CT % 2 == 0 ? CT / 2 : KGI == 0 ? CT : 0;
-  constexpr int MB0 = KG == 2 && CT % 2 == 0 ? KGI * (CT / 2) : 0;
+  // the two waves that use them (one column: by the first).
+  constexpr int MB = CT % 2 == 0 ? CT / 2 : KGI == 0 ? CT : 0;
+  constexpr int MB0 = CT % 2 == 0 ? KGI * (CT / 2) : 0;
   constexpr int LA = RT / 2, LB = MB * P::kNL;
   constexpr int W0 = mid_wait_count(0, 1, AD, NB, LA, LB), W1 = mid_wait_count(1, 1, AD, NB, LA, LB);
-  const int cg = KG == 1 ? wave : wave & 3, ntiles = a.n >> 4, steps = 2 * nbr;
+  const int cg = wave & 3, ntiles = a.n >> 4, steps = 2 * nbr;
   const int ct0 = (cb * M::kCG + cg) * OT;
   const uint8_t* wcol[MB > 0 ? MB : 1];
 #pragma unroll
@@ -86,7 +90,7 @@ __device__ __forceinline__ void mid_steps(const MidArgs& a, uint8_t* lds, int by
   mid_wait<AD * LA + (NB - 1) * LB>();
   __syncthreads();
   typename P::K kk[CT];
-  h8_t blo[NU][CT], bhi[NU][CT];
+  h8_t blo[CT], bhi[CT];
   {
     typename P::R r[CT];
 #pragma unroll
@@ -96,13 +100,11 @@ __device__ __forceinline__ void mid_steps(const MidArgs& a, uint8_t* lds, int by
     for (int c = 0; c < CT; ++c)
       P::consts(kk[c], r[c], lane);
 #pragma unroll
-    for (int ui = 0; ui < NU; ++ui)
-#pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        typename P::W w;
-        P::words(w, bl + c * P::kTB, ui + KGI, lane);
-        P::dequant(kk[c], w, ui + KGI, blo[ui][c], bhi[ui][c]);
-      }
+    for (int c = 0; c < CT; ++c) {
+      typename P::W w;
+      P::words(w, bl + c * P::kTB, KGI, lane);
+      P::dequant(kk[c], w, KGI, blo[c], bhi[c]);
+    }
   }
   uint32_t as = 0, bs = 0;  // ring slots of step t and of its block
   h8_t af[2][RT];
@@ -128,93 +130,94 @@ __device__ __forceinline__ void mid_steps(const MidArgs& a, uint8_t* lds, int by
       __syncthreads();  // step t's operands of every wave landed; step t - 1 fully read
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t an = as == 0 ? NS - 1 : as - 1;  // slot of step t - 1
-      if (t + AD < steps)
-        issue_a(t + AD, an);
-      if (hh == 1 && b + NB < nbr)
-        issue_b(b + NB, bs);
       const uint32_t bsn = hh == 0 ? bs : bs + 1 == NB ? 0 : bs + 1;  // B slot of step t + 1
       const uint8_t* const al = lds + as * M::kASlot + KGI * 2 * RT * 1024 + 16 * lane;
       const uint32_t asn = as + 1 == NS ? 0 : as + 1;
       const uint8_t* const aln = lds + asn * M::kASlot + KGI * 2 * RT * 1024 + 16 * lane;
       const uint8_t* const bn = bl + bsn * M::kBSlot;
-      __builtin_amdgcn_sched_barrier(0);
       typename P::R r[CT];
-      if (hh == 1) {
+      typename P::W wv[CT];
+      h8_t nlo[CT], nhi[CT];
+      auto issue = [&] {
+        if (t + AD < steps)
+          issue_a(t + AD, an);
+        if (hh == 1 && b + NB < nbr)
+          issue_b(b + NB, bs);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        // The MFMAs on the low- or high-nibble fragments, under them the reads
+        // of the next A fragments (the next step's first ones at the end) and
+        // half of the next step's dequantisation.
+        if (h == 0) {
+          if (!kLate)
+            issue();
+#pragma unroll
+          for (int c = 0; c < CT; ++c) {
+            if (hh == 1)
+              P::raw(r[c], bn + c * P::kTB, lane);
+            P::words(wv[c], bn + c * P::kTB, 2 * (1 - hh) + KGI, lane);
+          }
+        }
+        const uint8_t* const src = h == 0 ? al + 1024 : aln;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+          af[1 - h][rt] = *reinterpret_cast<const h8_t*>(src + 2 * rt * 1024);
 #pragma unroll
         for (int c = 0; c < CT; ++c)
-          P::raw(r[c], bn + c * P::kTB, lane);
-      }
-      typename P::W wv[NU][CT];
-#pragma unroll
-      for (int ui = 0; ui < NU; ++ui)
-#pragma unroll
-        for (int c = 0; c < CT; ++c)
-          P::words(wv[ui][c], bn + c * P::kTB, 2 * (1 - hh) + ui + KGI, lane);
-      h8_t nlo[NU][CT], nhi[NU][CT];
-#pragma unroll
-      for (int ui = 0; ui < NU; ++ui) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          // The A fragments of the next group of MFMAs, the next step's
-          // first at the end.
-          const int i = 2 * ui + h, j = i + 1;
-          const uint8_t* const src = j < 2 * NU ? al + (j / 2 * 2 * RT + (j & 1)) * 1024 : aln;
 #pragma unroll
           for (int rt = 0; rt < RT; ++rt)
-            af[j & 1][rt] = *reinterpret_cast<const h8_t*>(src + 2 * rt * 1024);
+            acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h][rt], h ? bhi[c] : blo[c], acc[rt][c], 0, 0, 0);
 #pragma unroll
-          for (int c = 0; c < CT; ++c)
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-              acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[i & 1][rt], h ? bhi[ui][c] : blo[ui][c], acc[rt][c], 0, 0, 0);
-        }
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          if (hh == 1 && ui == 0)
+        for (int c = h * CT / 2; c < (h + 1) * CT / 2; ++c) {
+          if (hh == 1)
             P::consts(kk[c], r[c], lane);
-          P::dequant(kk[c], wv[ui][c], 2 * (1 - hh) + ui + KGI, nlo[ui][c], nhi[ui][c]);
+          P::dequant(kk[c], wv[c], 2 * (1 - hh) + KGI, nlo[c], nhi[c]);
+          asm volatile("" : "+v"(nlo[c]), "+v"(nhi[c]));  // formed in this step, under its MFMAs
         }
+        if (h == 0) {
+          if (hh == 1)
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * CT, 0);
+          else
+            __builtin_amdgcn_sched_group_barrier(0x100, CT, 0);
+        }
+#pragma unroll
+        for (int k = 0; k < RT * CT; ++k) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (k < RT)
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+          if (hh == 1)
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          else
+            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+        }
+        if (kLate)
+          __builtin_amdgcn_sched_barrier(0);
+        if (kLate && h == 0)
+          issue();
       }
 #pragma unroll
-      for (int ui = 0; ui < NU; ++ui)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) {
-          blo[ui][c] = nlo[ui][c];
-          bhi[ui][c] = nhi[ui][c];
-          asm volatile("" : "+v"(blo[ui][c]), "+v"(bhi[ui][c]));  // formed in this step, under its MFMAs
-        }
+      for (int c = 0; c < CT; ++c) {
+        blo[c] = nlo[c];
+        bhi[c] = nhi[c];
+      }
       as = asn;
       bs = bsn;
-      // The raw words first, then each MFMA followed by an LDS read (the
-      // next group's fragments) and vector work.
-      if (hh == 1)
-        __builtin_amdgcn_sched_group_barrier(0x100, CT + CT * NU, 0);
-      else
-        __builtin_amdgcn_sched_group_barrier(0x100, CT * NU, 0);
-#pragma unroll
-      for (int i = 0; i < 2 * NU * RT * CT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (i % (RT * CT) < RT)
-          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (hh == 1)
-          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
-        else
-          __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
-      }
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   mid_wait<0>();
 }
 
-template <class P, int RT, int CT, int KG, int NS, int NB, bool GATED>
+template <class P, int RT, int CT, int NS, int NB, bool GATED>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void mid_gemm_kernel(MidArgs a) {
-  using M = MidShape<P, RT, CT, KG, NS, NB>;
+  using M = MidShape<P, RT, CT, NS, NB>;
   constexpr int OT = GATED ? CT / 2 : CT;
   __shared__ __attribute__((aligned(16))) uint8_t lds[M::kLds];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int cg = KG == 1 ? wave : wave & 3, kg = KG == 1 ? 0 : wave >> 2;
+  const int cg = wave & 3, kg = wave >> 2;
   // Workgroup -> (row block, column block, K-slice).  Workgroup L runs on XCD
   // L % 8: the row blocks of one (column block, slice) share an XCD (its
   // weights), and slices are dealt so that an XCD reads few slices of x.
@@ -232,42 +235,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int c = 0; c < CT; ++c)
       acc[rt][c] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  if (KG == 1 || kg == 0)
-    mid_steps<P, RT, CT, KG, NS, NB, GATED, 0>(a, lds, by, cb, kb0, nbr, wave, lane, acc);
+  if (kg == 0)
+    mid_steps<P, RT, CT, NS, NB, GATED, 0>(a, lds, by, cb, kb0, nbr, wave, lane, acc);
   else
-    mid_steps<P, RT, CT, KG, NS, NB, GATED, KG - 1>(a, lds, by, cb, kb0, nbr, wave, lane, acc);
+    mid_steps<P, RT, CT, NS, NB, GATED, 1>(a, lds, by, cb, kb0, nbr, wave, lane, acc);
 
   // K-groups: each wave of a pair keeps half of the row tiles and takes the
   // other wave's sums of them (in either order the same two terms).
   f4_t sum[M::kHR][CT];
-  int rt_first = 0;
-  if constexpr (KG == 2) {
-    constexpr int H = RT / 2;
-    __syncthreads();  // every wave has read its last operands, and no load is in flight
-    f4_t* mine = reinterpret_cast<f4_t*>(lds) + wave * (H * CT * 64) + lane;
-    const f4_t* other = reinterpret_cast<const f4_t*>(lds) + (wave ^ 4) * (H * CT * 64) + lane;
+  constexpr int H = RT / 2;
+  __syncthreads();  // every wave has read its last operands, and no load is in flight
+  f4_t* mine = reinterpret_cast<f4_t*>(lds) + wave * (H * CT * 64) + lane;
+  const f4_t* other = reinterpret_cast<const f4_t*>(lds) + (wave ^ 4) * (H * CT * 64) + lane;
 #pragma unroll
-    for (int h = 0; h < H; ++h)
+  for (int h = 0; h < H; ++h)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
-        mine[(h * CT + c) * 64] = kg ? acc[h][c] : acc[H + h][c];
-        sum[h][c] = kg ? acc[H + h][c] : acc[h][c];
-      }
-    __syncthreads();
+    for (int c = 0; c < CT; ++c) {
+      mine[(h * CT + c) * 64] = kg ? acc[h][c] : acc[H + h][c];
+      sum[h][c] = kg ? acc[H + h][c] : acc[h][c];
+    }
+  __syncthreads();
 #pragma unroll
-    for (int h = 0; h < H; ++h)
+  for (int h = 0; h < H; ++h)
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
-        sum[h][c] += other[(h * CT + c) * 64];
-    rt_first = kg * H;
-  } else {
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        sum[rt][c] = acc[rt][c];
-  }
-  const int row_tile = by * RT + rt_first, live = (a.m + 15) >> 4;
+    for (int c = 0; c < CT; ++c)
+      sum[h][c] += other[(h * CT + c) * 64];
+  const int row_tile = by * RT + kg * H, live = (a.m + 15) >> 4;
   if (a.slices > 1) {
     // Slice sums in accumulator order: [slice][row tile][column tile][lane].
     const int wide = GATED ? 2 * ntiles : ntiles;
@@ -468,7 +461,7 @@ __global__ __launch_bounds__(256) void mid_reduce_kernel(MidArgs a) {
 
 template <class P, int RT, int CT, bool GATED>
 hipError_t mid_launch(hipStream_t s, MidArgs a) {
-  constexpr int KG = 2, kTiles = 4 * CT * P::kTB;
+  constexpr int kTiles = 4 * CT * P::kTB;
   // Ring depths that fit 160 KB: activations first (three slots of 32 KB, or
   // four of 16), then up to four blocks of weights.
   constexpr int NS = RT == 8 ? 3 : 4, kLeft = 160 * 1024 - NS * RT * 4096, NB = kLeft / kTiles < 4 ? kLeft / kTiles : 4;
@@ -482,7 +475,7 @@ hipError_t mid_launch(hipStream_t s, MidArgs a) {
   const DispatchEvents ev = dispatch_events();
   if (a.slices > 1)
     dispatch_events() = DispatchEvents{ev.start, nullptr};
-  (void)dispatch(mid_gemm_kernel<P, RT, CT, KG, NS, NB, GATED>, dim3((unsigned)grid), dim3(512), s, a);
+  (void)dispatch(mid_gemm_kernel<P, RT, CT, NS, NB, GATED>, dim3((unsigned)grid), dim3(512), s, a);
   if (a.slices > 1) {
     dispatch_events() = DispatchEvents{nullptr, ev.stop};
     (void)launch_mid_reduce(s, a, GATED);
