@@ -938,7 +938,7 @@ def main():
             "weight_bytes_per_step": dec["step_bytes"],
         },
         "roofline": {
-            "kernel": "q4k_gemv_gate_up_kernel (fused gate/up packing x in registers, M=8, K=4096, N=12288)",
+            "kernel": "decode_gemv_kernel (fused gate/up packing x in registers, M=8, K=4096, N=12288)",
             "bound": "hbm",
             "achieved": round(g["gbs"], 1),
             "peak": HBM_PEAK_GBS,

@@ -85,9 +85,9 @@ const char* q4k_last_error(void);
  * Weight keys its kernels on the type (forward.cpp:55-57).  Every type
  * serves q4k_linear, q4k_linear_norm, q4k_mlp_gate_up and q4k_mlp in every
  * phase.  Decode passes of a gated pair run one fused gate/up kernel for
- * Q4_K pairs, and for Q5_K and IQ4_XS pairs with m <= 8 and k = 4096 (the
- * types the reference fuses, fused_kernels.metal:44-200); other gated
- * decode passes (Q6_K, Q8_0, pairs of two types) make the reference's two
+ * Q4_K pairs, and for pairs of another type with m <= 8 and k = 4096 (the
+ * reference fuses Q5_K and IQ4_XS, fused_kernels.metal:44-200) or 9..63 rows;
+ * other gated decode passes (pairs of two types) make the reference's two
  * calls.  q4k_embedding and q4k_embedding_batch take Q4_K tables only
  * (Q4K_ETYPE otherwise). */
 int q4k_weight_create(const void* gguf_bytes, size_t bytes, uint32_t n, uint32_t k, uint32_t ggml_type, int device, q4k_weight** out);

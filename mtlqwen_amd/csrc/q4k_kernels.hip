@@ -1,6 +1,10 @@
 // Q4_K linear() kernels for gfx950 (MI355X / CDNA4), and the other GGUF
 // weight types on the same surface.
 //
+// Beside this file: q4k_decode.hip (decode_gemv_kernel: up to 8 rows, K = 4096),
+// q4k_rows.hip (rows_gemm_kernel: 9 to 63 rows) and q4k_mid.hip (mid_gemm_kernel
+// and stage_row_kernel: prefills too small to fill the CUs here).
+//
 //  stage_x_kernel, stage_gemm_kernel, stage_pack_kernel
 //                   activations -> fp16 operands with power-of-two scales
 //  q4k_gemv_kernel  staged decode GEMV (up to 48 rows), optionally gated
@@ -11,7 +15,7 @@
 //  q4k_gemm2_kernel, typed_gemm_kernel
 //                   pipelined prefill GEMMs on v_mfma_f32_16x16x32_f16
 //  gather_rows_kernel, relayout_kernel, typed_relayout_kernel
-//  embedding_kernel, embedding_batch_kernel, rms_norm_kernel
+//  embedding_kernel, embedding_batch_kernel, rms_norm_kernel, rms_norm8_kernel
 //                   the path's neighbours in a pass (token embedding
 //                   gather-dequant, RMS norm / LM-head rms_norm_gather)
 //
