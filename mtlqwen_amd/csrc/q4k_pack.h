@@ -127,7 +127,7 @@ constexpr int gu_wave_floats() {
 // of all 8 rows (one coalesced load per (block, row), lane l
 // holding elements 4l..4l+3; rows >= m read row 0 and are zeroed), calls
 // issue_first() once its x has landed, and turns its blocks into MFMA
-// operands in registers (through its LDS region).  NORM: x
+// operands in registers (through its LDS region; W = 8 or 16).  NORM: x
 // is RMS-normalised on the way in (native_ops.metal:6-40, the norm
 // forward.cpp:114 applies before the MLP): the W waves hold all of x between
 // them, so each row's sum of squares is their partial sums (ssq [wave][row])
@@ -175,25 +175,39 @@ __device__ __forceinline__ void gate_up_pack_x(const GemvArgs& a, float* xl, flo
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           ss[r] = fmaf(xv[j][r][e], xv[j][r][e], ss[r]);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1)
-        ss[r] += __shfl_xor(ss[r], off);
     }
-    if (lane < 8) {
-      float v = ss[0];
+    // The eight sums over the lanes by halving: a lane gives the other half of
+    // the rows it holds for its own, until lanes 8r .. 8r + 7 hold row r's (10
+    // shuffles; 48 with every lane summing every row).
 #pragma unroll
-      for (int r = 1; r < 8; ++r)
-        v = lane == r ? ss[r] : v;
-      ssq[wave][lane] = v;
+    for (int n = 4; n > 0; n >>= 1) {
+      const bool up = lane & (8 * n);
+#pragma unroll
+      for (int r = 0; r < n; ++r) {
+        const float give = up ? ss[r] : ss[r + n];
+        ss[r] = (up ? ss[r + n] : ss[r]) + __shfl_xor(give, 8 * n);
+      }
     }
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1)
+      ss[0] += __shfl_xor(ss[0], off);
+    if ((lane & 7) == 0)
+      ssq[wave][lane >> 3] = ss[0];
     __syncthreads();
+    // Row r's scale in lanes 8r .. 8r + 7, one square root and division for all.
+    // (With every sum and scale formed in every lane the norm took 5 us of a
+    // call; so 1.2: 8 rows of 4096 -> 1024 Q4_K 11.2 -> 7.5 us, Q6_K 11.5 -> 7.4.)
+    float tot = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; w += 8)
+      tot += ssq[w + (lane & 7)][lane >> 3];
+#pragma unroll
+    for (int off = 4; off > 0; off >>= 1)
+      tot += __shfl_xor(tot, off);
+    const int scales = __builtin_bit_cast(int, 1.0f / sqrtf(tot / (float)a.k + a.eps));
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      float tot = 0.0f;
-#pragma unroll
-      for (int w = 0; w < W; ++w)
-        tot += ssq[w][r];
-      const float scale = 1.0f / sqrtf(tot / (float)a.k + a.eps);
+      const float scale = __builtin_bit_cast(float, __builtin_amdgcn_readlane(scales, 8 * r));
 #pragma unroll
       for (int j = 0; j < BPW; ++j)
 #pragma unroll
