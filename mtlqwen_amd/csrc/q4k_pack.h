@@ -66,11 +66,19 @@ __device__ __forceinline__ void pack_x_regs(const float (&xv)[32], int lane, XBl
   for (int v = 0; v < 16; ++v) {
     const float t0 = xv[2 * v] * up, t1 = xv[2 * v + 1] * up;
     sum += t0 + t1;
-    // The high part truncated (its residual is exact in fp32), the low one
-    // rounded to nearest: no bias, and as fast as truncating both (rounding both
-    // to nearest took 0.5 us more of a call's 6.4).
-    const h2_t h = __builtin_bit_cast(h2_t, __builtin_amdgcn_cvt_pkrtz(t0, t1));
-    const h2_t l = h2_t{(_Float16)(t0 - (float)h[0]), (_Float16)(t1 - (float)h[1])};
+    // Both parts rounded to nearest, as the staging kernels round them: hi + lo
+    // then holds 23 significant bits of the larger elements, where a truncated
+    // hi leaves a residual of up to a whole ulp and lo drops one bit more (rows
+    // 4096 -> 1024, m = 8, against 64 bits: 1.69e-7, truncated 1.91e-7).  The
+    // opaque values keep hi at one v_cvt_pk_f16_f32, not converted again element
+    // by element for its residual, and the residuals in fp32 until theirs
+    // (4096 -> 1024, m = 8, Q6_K 5.97 us; truncated 6.13).
+    uint32_t hp = __builtin_bit_cast(uint32_t, h2_t{(_Float16)t0, (_Float16)t1});
+    asm("" : "+v"(hp));
+    const h2_t h = __builtin_bit_cast(h2_t, hp);
+    float l0 = t0 - (float)h[0], l1 = t1 - (float)h[1];
+    asm("" : "+v"(l0), "+v"(l1));
+    const h2_t l = h2_t{(_Float16)l0, (_Float16)l1};
     hw[v] = __builtin_bit_cast(uint32_t, h);
     lw[v] = __builtin_bit_cast(uint32_t, l);
   }

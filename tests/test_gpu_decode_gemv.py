@@ -72,3 +72,32 @@ def test_decode_gemv_gate_up(q4k, oracle, gpu, t, m, n, dtype):
     # Two projections' errors meet in each output; fp16 rounds gate, up and output.
     bar = 2e-5 if t in (TYPE_Q4_K, TYPE_Q5_K) else 1e-3
     assert row_rel_err(got, oracle.mlp_gate_up(x, wg, wu, n, K, ggml_type=t).astype(np.float32)) <= (2e-3 if dtype == torch.float16 else bar)
+
+
+def _picking_q4k(n, k):
+    """Q4_K bytes of the n x k matrix that has a single 1 per row (row r picks
+    element pick[r]) and zeros elsewhere: d = 1, scales 1, mins 0."""
+    pick = (np.arange(n, dtype=np.int64) * (k // n if k >= n else 1)) % k
+    w = np.zeros((n, k // 256, 144), dtype=np.uint8)
+    w[:, :, 0:2] = np.frombuffer(np.float16(1.0).tobytes(), dtype=np.uint8)
+    w[:, :, 4:8] = 1
+    w[:, :, 12:16] = 1
+    e = pick % 256
+    w[np.arange(n), pick // 256, 16 + 32 * (e // 64) + e % 32] = np.where(e % 64 < 32, 1, 16)
+    return w.reshape(-1), pick
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 4096, K), (8, 1024, K), (5, 12288, K), (8, 4096, 12288)])
+def test_activations_keep_23_bits(q4k, gpu, m, n, k):
+    """Rows of x picked one element per output: hi + lo, both rounded to
+    nearest, hold any value of 23 significant bits exactly, and no other term of
+    the sum is non-zero, so the outputs equal the activations bit for bit."""
+    rng = np.random.default_rng(8400 + m + n)
+    x = (rng.uniform(0.125, 1.0, (m, k)) * rng.choice([-1.0, 1.0], (m, k))).astype(np.float32)
+    x = (x.view(np.uint32) & np.uint32(0xFFFFFFFE)).view(np.float32)
+    w, pick = _picking_q4k(n, k)
+    W = q4k.Weight(w, n, k)
+    y = torch.full((m, n), float("nan"), device=gpu)
+    q4k.linear(torch.from_numpy(x).to(gpu), W, m, y, query_counts=[1] * m)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), x[:, pick])
