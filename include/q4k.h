@@ -17,12 +17,17 @@
  *  - Calls on one device share that device's staging workspace: issue them
  *    from one submitter / one stream at a time, as the reference engine does
  *    (single worker thread, one command buffer per pass).
- *  - The workspace grows (hipMalloc) on the first call of a larger shape and
- *    is kept until the process ends.  A call made while its stream captures
- *    a HIP graph must not need growth: the launch that would need it fails
- *    with Q4K_ECAPTURE before allocating (q4k_mlp and the two-call form of
- *    q4k_mlp_gate_up may have enqueued their earlier launches by then).  One
- *    call of the same shapes before the capture avoids it.
+ *  - The workspace lives until the process ends.  The first projection on a
+ *    device, of any shape, reserves about 93 MB (hipMalloc); a call that
+ *    needs more (mostly by staging more activations: m * k above 4.3 million,
+ *    m rounded up to 128) grows it.  Which kernel a call takes depends on its
+ *    shape alone, so a captured call gives the bits of the eager one.  A call
+ *    made while its stream captures a HIP graph must not need growth: the
+ *    launch that would need it fails with Q4K_ECAPTURE before allocating
+ *    (q4k_mlp and the two-call form of q4k_mlp_gate_up may have enqueued
+ *    their earlier launches by then).  One call of the same shapes, or (k
+ *    up to 32768) of the same weights with more rows, before the capture
+ *    avoids it.
  */
 #ifndef Q4K_H
 #define Q4K_H

@@ -87,6 +87,7 @@ struct Workspace {
   // Fixed-size buffers in the no-allocation scratch: never grown; a call
   // that needs more fails (ensure_buffer).
   bool fixed = false;
+  bool reserved = false;  // reserve_workspace has run
 };
 
 Workspace g_ws[64];
@@ -414,6 +415,39 @@ int ensure_splitk_workspace(hipStream_t stream, Workspace& ws, int device, size_
   return Q4K_OK;
 }
 
+// Longest row of the rows GEMM, and the fp16 values it stages: 128 rows, then
+// the sub-block sums, 256 values per block and row tile.
+constexpr uint32_t kRowsGemmMaxK = 32768;
+constexpr size_t rows_gemm_halves(size_t k) {
+  return 132 * k;
+}
+
+// Which kernel a call takes depends on its shape alone, never on what the
+// workspace holds, so that a captured call and an eager one give the same bits.
+// Kernels differ in the buffers they need (a prefill of 512 rows may sum no
+// K-slices where one of 64 sums sixteen), so a device's first call outside a
+// capture reserves what any call of up to 63 rows and any K-sliced one can need
+// (about 93 MB, once): a capture then grows nothing unless it stages more
+// activations than any call before it.  A card too full for it is not an
+// error here: the calls grow what they need themselves.
+void reserve_workspace(hipStream_t stream, Workspace& ws, int device) {
+  if (ws.reserved || ws.fixed || stream_capturing(stream))
+    return;
+  ws.reserved = true;
+  const std::string last = g_error;
+  int rc = ensure_workspace(stream, ws, device, rows_gemm_halves(kRowsGemmMaxK), 1024);
+  if (!rc)
+    rc = ensure_splitk_workspace(stream, ws, device, kMidPartFloats, 8192);
+  if (!rc)
+    rc = ensure_buffer(stream, ws, device, ws.pack, ws.pack_bytes, kRowsGemmMaxK / 256 * kPackBytesPerBlock, "decode pack");
+  if (!rc)
+    rc = ensure_buffer(stream, ws, device, ws.normed, ws.normed_bytes, (size_t)64 * kRowsGemmMaxK * sizeof(float), "normalised-activation buffer");
+  if (rc) {
+    (void)hipGetLastError();
+    g_error = last;
+  }
+}
+
 // The pipelined GEMM of a shape with fewer tiles than CUs runs two
 // K-segments per tile (gemm2_split_b): their accumulators and arrival
 // counters live in the split-K workspace.
@@ -496,12 +530,8 @@ int set_device(int device) {
 }
 
 // A prefill GEMM of the middle row counts (mid_plan): x staged as for the
-// other GEMMs, the K-slices' sums in the split-K workspace.  A capture that
-// finds the workspace too small takes one slice (no sums to hold) instead of
-// growing it.
-int run_mid(hipStream_t stream, Workspace& ws, q4k_weight* w, const GemmArgs& g, uint32_t dtype, MidPlan plan, bool gated) {
-  if (plan.slices > 1 && ws.part_elems < plan.part_floats && stream_capturing(stream))
-    plan.slices = 1;
+// other GEMMs, the K-slices' sums in the split-K workspace.
+int run_mid(hipStream_t stream, Workspace& ws, q4k_weight* w, const GemmArgs& g, uint32_t dtype, const MidPlan& plan, bool gated) {
   if (plan.slices > 1) {
     int rc = ensure_buffer(stream, ws, w->device, ws.part, ws.part_elems, plan.part_floats, "split-K workspace");
     if (rc)
@@ -625,13 +655,6 @@ int run_gemv_groups_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, con
 // the weights again: the Q6_K LM head (N = 248320) of 40 rows 262 us against
 // 803, the Q6_K / Q5_K 12288 -> 4096 projection of 19 rows 24 us against 66.
 // wu != nullptr: the fused gate/up pair (one type).
-constexpr uint32_t kRowsGemmMaxK = 32768;
-
-bool rows_gemm_fits(hipStream_t stream, const Workspace& ws, uint32_t m, uint32_t k, size_t part_floats) {
-  // A capture may not grow the workspace: it keeps the GEMV groups then.
-  return (ws.x_elems >= (size_t)128 * k + (size_t)4 * k && ws.scale && ws.part_elems >= part_floats) || ws.fixed || !stream_capturing(stream);
-}
-
 // K-slices that fill the CUs the column blocks leave idle, each at least two
 // blocks long.
 int rows_gemm_slices(uint32_t m, uint32_t n, uint32_t nb, bool gated, int cus) {
@@ -649,8 +672,7 @@ int run_rows_gemm_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_w
   MidArgs a;
   a.slices = rows_gemm_slices(m, w->n, w->k / 256, wu != nullptr, device_cus(w->device));
   const size_t part = a.slices > 1 ? (size_t)a.slices * ((m + 15) / 16 * 16) * w->n * (wu ? 2 : 1) : 0;
-  // 128 staged rows, then the sub-block sums: 256 halves per block and row tile.
-  int rc = ensure_workspace(stream, ws, w->device, (size_t)128 * w->k + (size_t)4 * w->k, 64);
+  int rc = ensure_workspace(stream, ws, w->device, rows_gemm_halves(w->k), 64);
   if (!rc && part)
     rc = ensure_buffer(stream, ws, w->device, ws.part, ws.part_elems, part, "split-K workspace");
   if (rc)
@@ -678,12 +700,9 @@ int run_rows_gemm_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_w
   return Q4K_OK;
 }
 
-// Whether 9..63 rows of this weight (pair) take the rows GEMM now.
-bool rows_gemm_takes(hipStream_t stream, const Workspace& ws, const q4k_weight* w, uint32_t m, bool gated) {
-  if (m <= 8 || m >= kTypedGemmRows || w->k > kRowsGemmMaxK)
-    return false;
-  const int s = rows_gemm_slices(m, w->n, w->k / 256, gated, device_cus(w->device));
-  return rows_gemm_fits(stream, ws, m, w->k, s > 1 ? (size_t)s * ((m + 15) / 16 * 16) * w->n * (gated ? 2 : 1) : 0);
+// Whether m rows of a weight (pair) of this k take the rows GEMM.
+bool rows_gemm_takes(uint32_t m, uint32_t k) {
+  return m > 8 && m < kTypedGemmRows && k <= kRowsGemmMaxK;
 }
 
 // Up to 8 rows with K = 4096, plain or (wu) a gate/up pair of one type: one
@@ -716,7 +735,7 @@ int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const voi
                      uint32_t dtype, const float* norm_w, float eps) {
   if (m >= kTypedGemmRows && w->n >= kGemmMinColumns)
     return run_typed_gemm_locked(stream, ws, w, x, y, aux, m, post, dtype, norm_w, eps);
-  if (rows_gemm_takes(stream, ws, w, m, false))
+  if (rows_gemm_takes(m, w->k))
     return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   if (decode_gemv_supported((int)m, (int)(w->k / 256), (int)w->n, false, device_cus(w->device)))
     return run_decode_gemv(stream, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
@@ -730,6 +749,7 @@ int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const voi
 // 114), folded into the activation staging where the path stages x.
 int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weight* wu, const void* x, void* y, const void* aux, uint32_t m,
                       uint32_t post, uint32_t dtype, uint32_t phase, bool restage, const float* norm_w = nullptr, float eps = 0.0f) {
+  reserve_workspace(stream, ws, w->device);
   if (w->type != Q4K_GGML_TYPE_Q4_K) {
     if (wu)
       return fail(Q4K_ETYPE, "the fused gate/up kernel takes Q4_K weights");
@@ -744,7 +764,7 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
   // against 233 on the staged GEMV, 24 194 / 335, 32 200 / 241, 40 240 / 346).
   // With fewer column blocks the staged and rows GEMVs are ahead (N = 4096, M
   // = 40: 12.3 us against 17.6; N = 12288: 23.9 against 26.0).
-  if (!wu && m <= 16u * kGemvMaxRowTiles && (int)(w->n / 16) >= 16 * device_cus(w->device) && rows_gemm_takes(stream, ws, w, m, false))
+  if (!wu && m <= 16u * kGemvMaxRowTiles && (int)(w->n / 16) >= 16 * device_cus(w->device) && rows_gemm_takes(m, w->k))
     return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   if (!wu && w->n < kGemmMinColumns && m > kGemvSplitRows) {
     int rc = prenorm(stream, ws, w->device, x, norm_w, eps, m, w->k, dtype);
@@ -1303,13 +1323,15 @@ int mlp_gate_up_impl(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x
     // fused_kernels.metal:80-200).
     Workspace& ws = workspace(wg->device);
     std::lock_guard<std::mutex> lock(ws.mu);
+    reserve_workspace(s, ws, wg->device);
     resolve(wg, phase);
     resolve(wu, phase);
     return run_decode_gemv(s, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, norm_w, eps);
   }
   Workspace& ws = workspace(wg->device);
   std::lock_guard<std::mutex> lock(ws.mu);
-  if (!q4 && wg->type == wu->type && rows_gemm_takes(s, ws, wg, m, true)) {
+  reserve_workspace(s, ws, wg->device);
+  if (!q4 && wg->type == wu->type && rows_gemm_takes(m, wg->k)) {
     resolve(wg, phase);
     resolve(wu, phase);
     return run_rows_gemm_locked(s, ws, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, norm_w, eps);

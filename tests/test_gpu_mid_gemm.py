@@ -3,9 +3,10 @@ K in slices over the idle CUs) against the CPU oracle, at the edges of their
 tiles: one row above and below the 64- and 128-row blocks, a last column block
 of one live tile, K of one to three blocks (one slice; slices of unequal
 length), every weight type, epilogue and activation type; the gated form
-against the two calls; a capture that may not grow the workspace.  Bar: max
-row-relative error 1e-3, the one fp16 rounding of the activations and of the
-tile weights (2^-11 each) over at least 256 outputs of a row."""
+against the two calls; a capture after the same call (test_gpu_capture.py has
+those after other calls).  Bar: max row-relative error 1e-3, the one fp16
+rounding of the activations and of the tile weights (2^-11 each) over at least
+256 outputs of a row."""
 import numpy as np
 import pytest
 import torch
