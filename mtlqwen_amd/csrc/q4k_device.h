@@ -40,14 +40,21 @@ __device__ __forceinline__ void store_elem(T* p, size_t i, float v) {
   p[i] = (T)v;
 }
 
+// Vectors at addresses that a caller gives, aligned to one element only: the
+// backend emits the same 8- and 16-byte loads for them (global memory accesses
+// need no alignment on this target), but may assume nothing from the address.
+typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 h4_any_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef _Float16 h8_any_t __attribute__((ext_vector_type(8), aligned(2)));
+
 // Loads 8 consecutive activations as fp32.
 __device__ __forceinline__ void load8(const float* p, float* v) {
-  f4_t a = *reinterpret_cast<const f4_t*>(p), b = *reinterpret_cast<const f4_t*>(p + 4);
+  f4_t a = *reinterpret_cast<const f4_any_t*>(p), b = *reinterpret_cast<const f4_any_t*>(p + 4);
   v[0] = a[0], v[1] = a[1], v[2] = a[2], v[3] = a[3], v[4] = b[0], v[5] = b[1], v[6] = b[2], v[7] = b[3];
 }
 
 __device__ __forceinline__ void load8(const _Float16* p, float* v) {
-  h8_t a = *reinterpret_cast<const h8_t*>(p);
+  h8_t a = *reinterpret_cast<const h8_any_t*>(p);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
     v[i] = (float)a[i];

@@ -154,12 +154,12 @@ __device__ __forceinline__ void gate_up_pack_x(const GemvArgs& a, float* xl, flo
     for (int r = 0; r < 8; ++r) {
       const OutT* p = reinterpret_cast<const OutT*>(a.x) + (size_t)(r < a.m ? r : 0) * a.k + (size_t)(bw + j) * 256 + 4 * lane;
       if (sizeof(OutT) == 4) {
-        const f4_t v4 = *reinterpret_cast<const f4_t*>(p);
+        const f4_t v4 = *reinterpret_cast<const f4_any_t*>(p);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           xv[j][r][e] = v4[e];
       } else {
-        const h4_t v4 = *reinterpret_cast<const h4_t*>(p);
+        const h4_t v4 = *reinterpret_cast<const h4_any_t*>(p);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           xv[j][r][e] = (float)v4[e];
@@ -169,7 +169,7 @@ __device__ __forceinline__ void gate_up_pack_x(const GemvArgs& a, float* xl, flo
   if constexpr (NORM) {
 #pragma unroll
     for (int j = 0; j < BPW; ++j)
-      nw[j] = *reinterpret_cast<const f4_t*>(a.norm_w + (size_t)(bw + j) * 256 + 4 * lane);
+      nw[j] = *reinterpret_cast<const f4_any_t*>(a.norm_w + (size_t)(bw + j) * 256 + 4 * lane);
   }
   __builtin_amdgcn_sched_barrier(0);
 
