@@ -3079,10 +3079,20 @@ static int split_segments_per_wg(int tiles, int cus) {
 //    us for b = 10..13 against 64.3 unsplit: the segments 0 run at 5.4 us
 //    per block against 4.0 unsplit, so that 252 workgroups gain only 8 %
 //    over 168.
-//  - q >= 3: no split.  The few free CUs then hold q short segments each, whose
+//  - q = 3, K >= 8192, N < K and the free CUs at least 7/8 filled (192 tiles on
+//    256 CUs): b as for q = 2.  K = 12288 -> N = 4096 at M = 1536 170.1-172.0
+//    us against 177.2-178.0 unsplit, K = 12288 -> 8192 at M = 768 163.9
+//    against 176.4, K = 8192 -> 4096 at M = 1536 119.8 against 123.6.  Less
+//    filled it gains nothing (176 tiles, M = 1408: 168.2-172.7 against
+//    159.9-173.4), and neither does K = 4096 (-> 4096, M = 1536: 71.4
+//    against 68.5).  A gate/up pair takes the same b (its bits are the two
+//    calls') and loses by it (8192 -> 8192 at M = 768 276 us against 232):
+//    pairs widen, so the rule keeps to projections that narrow.
+//  - Otherwise no split.  The few free CUs then hold q short segments each, whose
 //    exchanges follow one another: N = 12288 at M = 640 (q = 15) measured 182
 //    us against 77.7 unsplit, its gate/up pair 251 against 139; N = 8192 at
-//    M = 821 (q = 7) 102 against 73.2, at M = 705 (q = 3) 69.1 against 67.9.
+//    M = 821 (q = 7) 102 against 73.2; K = 12288 -> 4096 at M = 1700 (q = 7)
+//    215 against 197, at M = 1920 (q = 15) 273 against 206.
 // Returns b, or 0 for no split.  Q4K_GEMM2_SPLIT=0 turns the split off;
 // Q4K_GEMM2_SPLIT_B forces b (for every shape with tiles < CUs and b < nb).
 int gemm2_split_b(int m, int n, int nb, int cus) {
@@ -3096,7 +3106,8 @@ int gemm2_split_b(int m, int n, int nb, int cus) {
   const int q = split_segments_per_wg(tiles, cus);
   if (q == 1)
     return nb >= 32 ? nb / 2 : 0;
-  return q == 2 && nb >= 16 ? (q * nb + q) / (q + 1) : 0;
+  const bool three = q == 3 && nb >= 32 && n < 256 * nb && 8 * tiles >= 21 * (cus - tiles);
+  return (q == 2 && nb >= 16) || three ? (q * nb + q) / (q + 1) : 0;
 }
 
 void gemm2_split_workspace(int m, int n, bool gated, size_t* part_floats, size_t* counters) {

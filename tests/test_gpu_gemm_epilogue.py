@@ -52,3 +52,29 @@ def test_gated_epilogue(q4k, gpu, shift):
     q4k.mlp_gate_up(x, G, U, m, y2, query_counts=[m])
     torch.cuda.synchronize()
     assert torch.isfinite(y2).all() and torch.equal(y1, y2)
+
+
+@pytest.mark.parametrize("m,n,k,post", [(1500, 4096, 8192, 1), (1536, 4080, 8448, 0), (1408, 4096, 8192, 2)])
+def test_narrowing_projection_in_segments(q4k, oracle, gpu, m, n, k, post):
+    """Long K in two K-segments of unequal length, the short ones three to a
+    workgroup (192 tiles on 256 CUs; 176 tiles stay whole): sampled rows against
+    the oracle, the same bits from one call to the next (the segments' exchange),
+    and the pair's one launch against the two calls."""
+    rng = np.random.default_rng(7950 + m)
+    w = make_q4k(rng, n, k)
+    x, aux = make_x(rng, m, k, 0.1), make_x(rng, m, n, 2.0)
+    W, U = q4k.Weight(w, n, k), q4k.Weight(make_q4k(rng, n, k), n, k)
+    xt, at = torch.from_numpy(x).to(gpu), torch.from_numpy(aux).to(gpu)
+    ys = [torch.full((m, n), float("nan"), device=gpu) for _ in range(3)]
+    for y in ys:
+        q4k.linear(xt, W, m, y, auxiliary=at if post else None, gated=post == 2, query_counts=[m])
+    torch.cuda.synchronize()
+    assert torch.equal(ys[0], ys[1]) and torch.equal(ys[0], ys[2])
+    rows = np.r_[0:m:149, m - 1]
+    ref = oracle.linear(x[rows], w, n, k, aux=aux[rows] if post else None, post=post)
+    assert row_rel_err(ys[0].cpu().numpy()[rows], ref) <= TOL
+    q4k.linear(xt, W, m, ys[0], query_counts=[m])
+    q4k.linear(xt, U, m, ys[0], auxiliary=ys[0], gated=True, query_counts=[m])
+    q4k.mlp_gate_up(xt, W, U, m, ys[1], query_counts=[m])
+    torch.cuda.synchronize()
+    assert torch.equal(ys[0], ys[1])
