@@ -700,9 +700,20 @@ int run_rows_gemm_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_w
   return Q4K_OK;
 }
 
-// Whether m rows of a weight (pair) of this k take the rows GEMM.
-bool rows_gemm_takes(uint32_t m, uint32_t k) {
-  return m > 8 && m < kTypedGemmRows && k <= kRowsGemmMaxK;
+// Whether m rows of a weight (wu: a pair) take the rows GEMM.  Up to 16 plain
+// rows of a short K whose column tiles fit one round of the CUs keep the GEMV
+// groups for the types with the costlier block constants: two passes over few
+// weights take less than the K-slices' reduction launch (16 rows, rows GEMM
+// against groups: Q6_K 1024 -> 1024 10.2 / 9.8 us, 2048 -> 512 11.3 / 10.7,
+// IQ4_XS 1024 -> 1024 10.6 / 9.8, 2048 -> 2048 11.7 / 11.0; Q8_0 10.6 / 11.2 and
+// Q5_K 11.4 / 11.7 at 2048 -> 1024 and -> 2048, Q6_K at K = 512 8.6 / 9.1,
+// 2304 -> 1024 12.3 / 12.0, 3072 -> 1024 11.5 / 12.9, 2048 -> 8192 14.0 / 17.4).
+// A norm would be a launch of its own there.
+bool rows_gemm_takes(const q4k_weight* w, bool gated, uint32_t m, bool norm) {
+  if (m <= 8 || m >= kTypedGemmRows || w->k > kRowsGemmMaxK)
+    return false;
+  const bool costly = w->type == Q4K_GGML_TYPE_Q6_K || w->type == Q4K_GGML_TYPE_IQ4_XS;
+  return gated || norm || !costly || m > 16 || w->k < 768 || w->k > 2304 || (int)(w->n / 16) > device_cus(w->device);
 }
 
 // Up to 8 rows with K = 4096, plain or (wu) a gate/up pair of one type: one
@@ -735,7 +746,7 @@ int run_typed_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, const voi
                      uint32_t dtype, const float* norm_w, float eps) {
   if (m >= kTypedGemmRows && w->n >= kGemmMinColumns)
     return run_typed_gemm_locked(stream, ws, w, x, y, aux, m, post, dtype, norm_w, eps);
-  if (rows_gemm_takes(m, w->k))
+  if (rows_gemm_takes(w, false, m, norm_w != nullptr))
     return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   if (decode_gemv_supported((int)m, (int)(w->k / 256), (int)w->n, false, device_cus(w->device)))
     return run_decode_gemv(stream, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
@@ -764,7 +775,7 @@ int run_linear_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, q4k_weig
   // against 233 on the staged GEMV, 24 194 / 335, 32 200 / 241, 40 240 / 346).
   // With fewer column blocks the staged and rows GEMVs are ahead (N = 4096, M
   // = 40: 12.3 us against 17.6; N = 12288: 23.9 against 26.0).
-  if (!wu && m <= 16u * kGemvMaxRowTiles && (int)(w->n / 16) >= 16 * device_cus(w->device) && rows_gemm_takes(m, w->k))
+  if (!wu && m <= 16u * kGemvMaxRowTiles && (int)(w->n / 16) >= 16 * device_cus(w->device) && rows_gemm_takes(w, false, m, norm_w != nullptr))
     return run_rows_gemm_locked(stream, ws, w, nullptr, x, y, aux, m, post, dtype, norm_w, eps);
   if (!wu && w->n < kGemmMinColumns && m > kGemvSplitRows) {
     int rc = prenorm(stream, ws, w->device, x, norm_w, eps, m, w->k, dtype);
@@ -1331,7 +1342,7 @@ int mlp_gate_up_impl(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x
   Workspace& ws = workspace(wg->device);
   std::lock_guard<std::mutex> lock(ws.mu);
   reserve_workspace(s, ws, wg->device);
-  if (!q4 && wg->type == wu->type && rows_gemm_takes(m, wg->k)) {
+  if (!q4 && wg->type == wu->type && rows_gemm_takes(wg, true, m, norm_w != nullptr)) {
     resolve(wg, phase);
     resolve(wu, phase);
     return run_rows_gemm_locked(s, ws, wg, wu, x, y, nullptr, m, Q4K_POST_STORE, dtype, norm_w, eps);

@@ -86,3 +86,24 @@ def test_rows_gemm_capture(q4k, gpu):
         torch.cuda.synchronize()
         assert torch.equal(y, y_ref)
         q4k.linear(x * 0.5, W, m, torch.empty_like(y), query_counts=[m])
+
+
+@pytest.mark.parametrize("t,m,n,k,launches", [(TYPE_Q6_K, 16, 1024, 1024, 2), (TYPE_IQ4_XS, 9, 4096, 2048, 2), (TYPE_Q6_K, 12, 256, 768, 2),
+                                              (TYPE_Q6_K, 17, 1024, 1024, 1), (TYPE_IQ4_XS, 16, 256, 512, 1), (TYPE_IQ4_XS, 9, 144, 2304, 2), (TYPE_Q6_K, 16, 144, 2560, 1),
+                                              (TYPE_IQ4_XS, 16, 4112, 2048, 1), (TYPE_Q5_K, 16, 1024, 1024, 1), (TYPE_Q8_0, 16, 512, 2048, 1)])
+def test_few_rows_of_short_k(q4k, oracle, gpu, t, m, n, k, launches):
+    """9 to 16 rows at the edges of the sizes that keep one GEMV per 8 rows:
+    `launches` of the GEMV family."""
+    rng = np.random.default_rng(7800 + m + n + k)
+    w = make_weight(rng, n, k, t)
+    W = q4k.Weight(w, n, k, ggml_type=t)
+    x = make_x(rng, m, k, 0.25)
+    y, xt = torch.full((m, n), float("nan"), device=gpu), torch.from_numpy(x).to(gpu)
+    torch.cuda.synchronize()
+    q4k.profile_enable(True)
+    q4k.linear(xt, W, m, y, query_counts=[m])
+    torch.cuda.synchronize()
+    got = q4k.profile_query(q4k.KERNEL_GEMV)[0]
+    q4k.profile_enable(False)
+    assert got == launches
+    assert row_rel_err(y.cpu().numpy(), oracle.linear(x, w, n, k, ggml_type=t)) <= _bar(t, torch.float32)
