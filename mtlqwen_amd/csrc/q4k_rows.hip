@@ -18,7 +18,7 @@ namespace {
 // sums of the block; kMin: the min term, dmin times the 16x16x16 MFMA of the
 // sub-block sums with bmin (32 m_j; k = 0..7 the hi parts, 8..15 the lo ones).
 struct RxQ4K : TgQ4K {
-  static constexpr bool kFold = true, kMin = true;
+  static constexpr bool kFold = true, kMin = true, kShortSums = true;
   struct K {
     float d, dmin;
     h2_t mul_lo, add_lo, mul_hi, add_hi;
@@ -48,7 +48,7 @@ struct RxQ4K : TgQ4K {
 };
 
 struct RxQ5K : TgQ5K {
-  static constexpr bool kFold = true, kMin = true;
+  static constexpr bool kFold = true, kMin = true, kShortSums = false;
   struct K : RxQ4K::K {
     uint32_t h0, h1;
   };
@@ -75,7 +75,7 @@ struct RxQ5K : TgQ5K {
 };
 
 struct RxQ6K : TgQ6K {
-  static constexpr bool kFold = true, kMin = false;
+  static constexpr bool kFold = true, kMin = false, kShortSums = false;
   struct K {
     float d, dmin;
     h2_t mul[4], add[4];  // of scale byte i: sc / 16 and -96 sc
@@ -118,7 +118,7 @@ struct RxQ6K : TgQ6K {
 };
 
 struct RxQ8_0 : TgQ8_0 {
-  static constexpr bool kFold = false, kMin = false;  // q * d, rounded once to fp16
+  static constexpr bool kFold = false, kMin = false, kShortSums = false;  // q * d, rounded once to fp16
   struct K : TgQ8_0::K {
     float d, dmin;
   };
@@ -131,7 +131,7 @@ struct RxQ8_0 : TgQ8_0 {
 };
 
 struct RxIQ4XS : TgIQ4XS {
-  static constexpr bool kFold = true, kMin = false;
+  static constexpr bool kFold = true, kMin = false, kShortSums = false;
   struct K {
     float d, dmin;
     h2_t mul0, add0, mul1, add1;  // ls - 32 and -1152 (ls - 32) of sub-blocks 2g, 2g + 1
@@ -267,7 +267,15 @@ __device__ __forceinline__ void rows_run(const MidArgs& a, uint8_t* lds, int wav
     P::words(w, bl + c * P::kTB, KGI, lane);
     P::frags(kk[c], w, KGI, blo[c], bhi[c]);
   }
-  f4_t acc[RT][CT], blk[RT][CT];
+  // Up to 32 rows of Q4_K (kShortSums): fp32 sums of four blocks at a time, and a
+  // step's low parts before its high ones, so that no sum runs over all of K in
+  // full size: N = 66048, K = 4096 against 64 bits 1.80e-7, in one run 2.15e-7;
+  // the staged GEMV, whose waves sum one or two blocks, 1.82e-7 (times even:
+  // N = 248320, 9 rows 166 against 162 us, 24 rows 207 against 208).  The other
+  // types' sums are already closer than the GEMV groups' that they replace
+  // (Q5_K 1.94e-7 against 2.05e-7).
+  constexpr bool SHORT = P::kShortSums && RT <= 2;
+  f4_t acc[RT][CT], blk[RT][CT], far[SHORT ? RT : 1][CT];
   uint32_t as = 0, bs = 0;
   int t = 0, xslot = 0;
   for (int it = 0; it < mine; ++it) {
@@ -276,6 +284,13 @@ __device__ __forceinline__ void rows_run(const MidArgs& a, uint8_t* lds, int wav
 #pragma unroll
       for (int c = 0; c < CT; ++c)
         acc[rt][c] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (SHORT) {
+#pragma unroll
+      for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+          far[rt][c] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
     for (int b = 0; b < nbr; ++b) {
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh, ++t) {
@@ -312,21 +327,22 @@ __device__ __forceinline__ void rows_run(const MidArgs& a, uint8_t* lds, int wav
 #pragma unroll
         for (int v = 0; v < VT; ++v)
           af[1][v] = *reinterpret_cast<const h8_t*>(al + (2 * v + 1) * 1024);
-        // hi then lo parts of every row tile, low- then high-nibble fragments.
+        // hi then lo parts of every row tile, low- then high-nibble fragments
+        // (SHORT: lo parts first, then hi).
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int i = 0; i < 4; ++i) {
+          const int h = SHORT ? i & 1 : i >> 1, p = SHORT ? 1 - (i >> 1) : i & 1;
 #pragma unroll
-          for (int p = 0; p < 2; ++p)
+          for (int c = 0; c < CT; ++c)
 #pragma unroll
-            for (int c = 0; c < CT; ++c)
-#pragma unroll
-              for (int rt = 0; rt < RT; ++rt) {
-                if constexpr (P::kFold)
-                  blk[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                      af[h][2 * rt + p], h ? bhi[c] : blo[c], hh == 0 && h == 0 && p == 0 ? f4_t{0.0f, 0.0f, 0.0f, 0.0f} : blk[rt][c], 0, 0, 0);
-                else
-                  acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h][2 * rt + p], h ? bhi[c] : blo[c], acc[rt][c], 0, 0, 0);
-              }
+            for (int rt = 0; rt < RT; ++rt) {
+              if constexpr (P::kFold)
+                blk[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h][2 * rt + p], h ? bhi[c] : blo[c],
+                                                                    hh == 0 && i == 0 ? f4_t{0.0f, 0.0f, 0.0f, 0.0f} : blk[rt][c], 0, 0, 0);
+              else
+                acc[rt][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h][2 * rt + p], h ? bhi[c] : blo[c], acc[rt][c], 0, 0, 0);
+            }
+        }
         float d[CT], dmin[CT];
         h4_t bmin[CT];
 #pragma unroll
@@ -371,6 +387,17 @@ __device__ __forceinline__ void rows_run(const MidArgs& a, uint8_t* lds, int wav
         __builtin_amdgcn_sched_barrier(0);
       }
       ++xslot;
+      if constexpr (SHORT) {
+        if ((b & 3) == 3 || b + 1 == nbr) {
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+              far[rt][c] += acc[rt][c];
+              acc[rt][c] = b + 1 == nbr ? far[rt][c] : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+      }
     }
     // The two K-groups' sums, two row tiles at a time: of the pair the wave of
     // K-group 0 finishes the even row tile, that of K-group 1 the odd one.

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from q4k_ref import TYPE_IQ4_XS, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0, make_weight, make_x, row_rel_err
+from q4k_ref import TYPE_IQ4_XS, TYPE_Q4_K, TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0, dequant_numpy, make_q4k, make_weight, make_x, row_rel_err
 
 pytestmark = pytest.mark.gpu
 TYPES = [TYPE_Q5_K, TYPE_Q6_K, TYPE_Q8_0, TYPE_IQ4_XS]
@@ -107,3 +107,63 @@ def test_few_rows_of_short_k(q4k, oracle, gpu, t, m, n, k, launches):
     q4k.profile_enable(False)
     assert got == launches
     assert row_rel_err(y.cpu().numpy(), oracle.linear(x, w, n, k, ggml_type=t)) <= _bar(t, torch.float32)
+
+
+def _first_wide():
+    """The fewest Q4_K outputs that take the rows GEMM (16 column tiles per CU), and a tile."""
+    return 16 * (16 * torch.cuda.get_device_properties(0).multi_processor_count + 1)
+
+
+@pytest.mark.parametrize("m,k,post,dtype", [(9, 512, 0, torch.float32), (17, 256, 1, torch.float32), (32, 768, 2, torch.float16), (33, 1280, 2, torch.float32),
+                                            (48, 512, 1, torch.float16), (48, 512, 0, torch.float32), (49, 512, 0, torch.float32)])
+def test_wide_q4k(q4k, oracle, gpu, m, k, post, dtype):
+    """Wide Q4_K outputs, several items to a workgroup and a last column block
+    of one tile: 9 to 48 rows on the rows GEMM (beyond 24 rows only it keeps 22
+    bits of the activations), 49 on the prefill GEMM."""
+    n = _first_wide()
+    rng = np.random.default_rng(7900 + m + k)
+    npdt = np.float16 if dtype == torch.float16 else np.float32
+    w = make_q4k(rng, n, k)
+    x = make_x(rng, m, k, 0.05).astype(npdt)
+    aux = make_x(rng, m, n, 2.0).astype(npdt) if post else None
+    W = q4k.Weight(w, n, k)
+    y = torch.from_numpy(aux).to(gpu) if post else torch.full((m, n), float("nan"), device=gpu, dtype=dtype)
+    xt = torch.from_numpy(x).to(gpu)
+    torch.cuda.synchronize()
+    q4k.profile_enable(True)
+    q4k.linear(xt, W, m, y, auxiliary=y if post else None, gated=post == 2, query_counts=[m])
+    torch.cuda.synchronize()
+    launches = [q4k.profile_query(f)[0] for f in (q4k.KERNEL_STAGE, q4k.KERNEL_GEMV, q4k.KERNEL_GEMM)]
+    q4k.profile_enable(False)
+    assert launches == ([1, 1, 0] if m <= 48 else [1, 0, 1])
+    got = y.float().cpu().numpy()
+    assert np.all(np.isfinite(got))
+    ref = oracle.linear(x, w, n, k, aux=aux, post=post).astype(np.float32)
+    assert row_rel_err(got, ref) <= (1e-3 if dtype == torch.float16 or m > 48 else 1e-5)
+
+
+@pytest.mark.parametrize("m", [9, 24])
+def test_wide_q4k_sums(q4k, gpu, m):
+    """The error against 64 bits of a wide Q4_K projection's first outputs is
+    that of the same rows of a narrow one (the staged GEMV, whose waves sum one
+    or two blocks each), within 5 %: both keep hi/lo activations, and the sums
+    over all of K in one workgroup are made as short.  Weights about zero, as
+    trained ones: the unsigned quants' part and the min part of a sum are each
+    larger than the result."""
+    n, narrow, k = _first_wide(), 2048, 4096
+    rng = np.random.default_rng(7950)
+    w = rng.integers(0, 256, (n, k // 256, 144), dtype=np.uint8)
+    d = ((0.5 + rng.random((n, k // 256, 1))) / 21760.0).astype(np.float16)
+    w[:, :, :4] = np.concatenate([d, (7.5 * d.astype(np.float32)).astype(np.float16)], axis=2).view(np.uint8)
+    w = w.reshape(n, -1)
+    x = make_x(rng, m, k)
+    ref = x.astype(np.float64) @ dequant_numpy(w[:narrow], narrow, k).astype(np.float64).T
+    err = []
+    for rows in (n, narrow):
+        W = q4k.Weight(np.ascontiguousarray(w[:rows]), rows, k)
+        y = torch.empty((m, rows), device=gpu)
+        q4k.linear(torch.from_numpy(x).to(gpu), W, m, y, query_counts=[m])
+        torch.cuda.synchronize()
+        err.append(np.linalg.norm(y[:, :narrow].double().cpu().numpy() - ref) / np.linalg.norm(ref))
+    print("wide, narrow", err)
+    assert err[0] <= 1.05 * err[1], err
