@@ -487,7 +487,7 @@ hipError_t launch_mid(hipStream_t s, MidArgs a, uint32_t type, const MidPlan& pl
 
 // 1..64 rows staged as hi/lo pairs (launch_stage_rows with xs): y = post(x W^T)
 // or SiLU(x W^T) * (x Wu^T) with the decode GEMVs' precision, every weight
-// type; a.slices K-slices.
+// type (Q4_K: plain, up to 48 rows); a.slices K-slices.
 hipError_t launch_rows_gemm(hipStream_t s, const MidArgs& a, uint32_t type, bool gated, int cus);
 
 // One MFMA-ceiling launch: `blocks` workgroups of 4 waves, each wave issuing

@@ -482,7 +482,9 @@ hipError_t rows_launch_rt(hipStream_t s, const MidArgs& a, int cus) {
     case 3:
       return rows_launch<P, 3, GATED>(s, a, cus);
     case 4:
-      return rows_launch<P, 4, GATED>(s, a, cus);
+      if constexpr (!P::kShortSums)  // Q4_K comes with at most 48 rows
+        return rows_launch<P, 4, GATED>(s, a, cus);
+      [[fallthrough]];
     default:
       return hipErrorInvalidValue;
   }
@@ -500,7 +502,8 @@ hipError_t launch_rows_gemm(hipStream_t s, const MidArgs& a, uint32_t type, bool
     return hipErrorInvalidValue;
   switch (type) {
     case kTypeQ4_K:
-      return rows_launch_any<RxQ4K>(s, a, gated, cus);
+      // Q4_K pairs take the decode and rows GEMVs.
+      return gated ? hipErrorInvalidValue : rows_launch_rt<RxQ4K, false>(s, a, cus);
     case kTypeQ5_K:
       return rows_launch_any<RxQ5K>(s, a, gated, cus);
     case kTypeQ6_K:
