@@ -4,8 +4,8 @@ reference's two-call form (forward.cpp:116-118: gate stored with post 0, then
 up with post 2 over it in place) run through linear(): the same buffer bit for
 bit, one GEMM launch instead of two, and the oracle on every row.  Cases: ragged row blocks and column blocks (a
 workgroup with one live output tile), one block of K, fp16 activations, the
-config-4 shape, long K with few tiles (two K-halves per tile, summed by the
-second half to finish), and the ffn_norm folded into the shared staging.
+config-4 shape, long K with few tiles, and the ffn_norm folded into the shared
+staging.
 Bar for the oracle: max row-relative error 1e-3, or, in rows where SiLU(gate)
 * up is ill-conditioned, no further from the oracle than the reference's own
 prefill arithmetic (see test_gated_gemm_matches_two_calls)."""
@@ -28,9 +28,10 @@ def _gemm_launches(q4k, fn):
     return n
 
 
-# (m, n, k, dtype): n = 1296 and 272 leave the last 128-column workgroup one
-# live output tile; k = 256 is one block; k = 8192 and 12288 with few tiles
-# run as two K-halves per tile in both forms; at (821, 6144) the plain GEMM
+# (m, n, k, dtype): n = 1296 and 272 leave the last column block one live
+# output tile; k = 256 is one block; the first three, k = 256, 8192 and 12288
+# take the middle GEMM, both forms in the same K-slices
+# (test_gpu_pipelined_gemm.py has two K-halves per tile); at (821, 6144) the plain GEMM
 # takes 192 columns per workgroup (the typed template) and neither form
 # splits K; at (821, 5120, 4096) both split K at block 11 of 16, the plain
 # GEMM with its short segments two to a workgroup, the gated one (280 tiles)

@@ -14,7 +14,7 @@ upload (bit-identical to the host one); the gated projection (one fused
 launch for Q5_K and IQ4_XS in the decode phase, with and without the
 ffn_norm); a GGUF file;
 and, for every non-Q4_K type, prefill batches of 64 rows and more (the
-typed MFMA GEMM): M = 2048, ragged row and column tails (a workgroup with
+middle and the typed MFMA GEMM, by shape): M = 2048, ragged row and column tails (a workgroup with
 one live column tile, waves with none), one block of K, post 0 / 1 / 2 and
 fp16 activations, and one-hot rows that read single dequantised weights
 out, which must equal the oracle's fp32 value rounded to fp16 exactly.
@@ -180,9 +180,9 @@ def test_tensor_from_gguf(q4k, oracle, gpu, tmp_path, t):
 # order (fp16, power-of-two row scales), the type's MFMA GEMM dequantising
 # each weight to the reference's prefill tile value (fp16) in registers.  Like
 # the Q4_K GEMM, activations and weights are single fp16 (expected row errors
-# ~4e-4).  592 = 16 * 37 columns: the last workgroup has 5 live column tiles
-# (one wave with a single tile, Q8_0's 2-tile waves: one with one) and
-# waves with none.
+# ~4e-4).  592 = 16 * 37 columns: one live column tile in the last column
+# block.  These shapes take the middle GEMM on 256 CUs; test_gpu_pipelined_gemm.py
+# has the tilings of more rows.
 ALL_TYPES = TYPES + [14]
 
 
@@ -223,8 +223,9 @@ def test_prefill_gemm_epilogues(q4k, oracle, gpu, t, post, dtype):
 def test_prefill_gemm_dequant_bit_exact(q4k, oracle, gpu, t):
     """Row r of x is one-hot at element r of block r % nb, so y[r, j] is the
     fp16 weight the GEMM formed for (j, that element) times 1: every element
-    position of a block, over all blocks, in 592 columns (512 for Q4_K, whose
-    pipelined GEMM takes N in multiples of 256)."""
+    position of a block, over all blocks, in 592 columns (512 for Q4_K).  The
+    middle GEMM takes this shape (test_gpu_pipelined_gemm.py has the pipelined
+    ones)."""
     m, n, k = 256, 512 if t == 12 else 592, 2048
     nb = k // 256
     rng = np.random.default_rng(990 + t)
