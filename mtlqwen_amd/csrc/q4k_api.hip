@@ -652,9 +652,10 @@ int run_gemv_groups_locked(hipStream_t stream, Workspace& ws, q4k_weight* w, con
 // 9 to 63 rows of the other types (and of the wide Q4_K projections): x staged
 // once as hi/lo rows, then one GEMM over all rows with the group GEMV's
 // precision (rows_gemm_kernel), instead of one GEMV per 8 rows, each reading
-// the weights again: the Q6_K LM head (N = 248320) of 40 rows 262 us against
-// 803, the Q6_K / Q5_K 12288 -> 4096 projection of 19 rows 24 us against 66.
+// the weights again: the Q6_K LM head (N = 248320) of 40 rows 271 us against
+// 800, the Q6_K / Q5_K 12288 -> 4096 projection of 19 rows 24 us against 66.
 // wu != nullptr: the fused gate/up pair (one type).
+
 // K-slices that fill the CUs the column blocks leave idle, each at least two
 // blocks long.
 int rows_gemm_slices(uint32_t m, uint32_t n, uint32_t nb, bool gated, int cus) {

@@ -1,8 +1,8 @@
 // GEMMs of the middle row counts for gfx950: prefill passes too small to fill
 // the chip with 128 x 256 tiles.
 //
-//  mid_gemm_kernel    column tiles x K-slices over all CUs, weights from
-//                     global memory straight into registers
+//  mid_gemm_kernel    column tiles x K-slices over all CUs, activations and
+//                     weights through LDS-DMA rings
 //  mid_reduce_kernel  sums the K-slices and applies the epilogue
 #include <hip/hip_runtime.h>
 #include <stdlib.h>
@@ -11,7 +11,6 @@
 
 namespace q4k {
 namespace {
-
 
 // ---- the kernel --------------------------------------------------------------
 // y = post(x W^T) for row blocks of 16 RT rows.  Workgroup = 8 waves = 2
