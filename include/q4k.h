@@ -92,8 +92,8 @@ const char* q4k_last_error(void);
  * phase.  Decode passes of a gated pair run one fused gate/up kernel for
  * Q4_K pairs, and for pairs of another type with m <= 8 and k = 4096 (the
  * reference fuses Q5_K and IQ4_XS, fused_kernels.metal:44-200) or 9..63 rows;
- * other gated decode passes (pairs of two types) make the reference's two
- * calls.  q4k_embedding and q4k_embedding_batch take Q4_K tables only
+ * other gated decode passes (pairs of two types, other k) make the
+ * reference's two calls.  q4k_embedding and q4k_embedding_batch take Q4_K tables only
  * (Q4K_ETYPE otherwise). */
 int q4k_weight_create(const void* gguf_bytes, size_t bytes, uint32_t n, uint32_t k, uint32_t ggml_type, int device, q4k_weight** out);
 
@@ -129,9 +129,11 @@ int q4k_linear(void* stream, q4k_weight* w, const void* x, void* y, const void* 
  * k + eps) * norm_w, norm_w k fp32 values), the pair the decoder runs for the
  * attention input (forward.cpp:82 attn_norm, then the QKV projections
  * :86-87, :99).  The norm is folded into the activation staging of the
- * selected kernel (decode GEMV, prefill GEMM); paths that pack x inside the
- * GEMV (split-K, the wide persistent GEMV) normalise into the workspace
- * first.  Arguments otherwise as q4k_linear; aux must not be x. */
+ * selected kernel, or into its own packing of x (m <= 8, k = 4096, up to 16
+ * column tiles per CU), in fp32: the normalised rows are not rounded to the
+ * dtype.  Paths that take x from the caller (the split-K GEMV, the wide
+ * persistent GEMV, GEMVs per 8 rows) normalise into a workspace buffer of the
+ * dtype first.  Arguments otherwise as q4k_linear; aux must not be x. */
 int q4k_linear_norm(void* stream, q4k_weight* w, const float* norm_w, float eps, const void* x, void* y, const void* aux, uint32_t m,
                     const uint32_t* query_counts, uint32_t nqueries, uint32_t post, uint32_t dtype);
 
@@ -143,7 +145,8 @@ int q4k_linear_norm(void* stream, q4k_weight* w, const float* norm_w, float eps,
  * results as q4k_linear, but the workspace is a fixed 120 MiB device array
  * that each GPU the library runs on holds until the process ends: 2 MiB of
  * decode pack (m <= 8, k <= 61440), 64 MiB of split-K partials (the decode
- * split-K GEMV and the prefill GEMM's two K-segments), 4096 split-K
+ * split-K GEMV, the K-slices of the middle and rows GEMMs and the prefill
+ * GEMM's two K-segments), 4096 split-K
  * counters, 65536 row scales, and about 54 MiB of staged activations (e.g.
  * m * k <= 28.1 million for prefill, rows padded to 128).  A call needing
  * more fails with Q4K_ESHAPE and a message naming the buffer.  Every weight
@@ -174,8 +177,8 @@ int q4k_mlp_gate_up(void* stream, q4k_weight* wg, q4k_weight* wu, const void* x,
  * decoder passes x = hidden with the layer's ffn_norm; the norm runs inside
  * the fused gate/up GEMV (decode, m <= 8, k = 4096) or inside the activation
  * staging that the gate and up projections share (prefill GEMM, other
- * decode GEMVs); only paths that pack x inside the GEMV normalise into a
- * workspace buffer first.  The gate buffer must not overlap x or hidden; x
+ * decode GEMVs); the paths that take x from the caller normalise into a
+ * workspace buffer first, as for q4k_linear_norm.  The gate buffer must not overlap x or hidden; x
  * may equal hidden. */
 int q4k_mlp(void* stream, q4k_weight* wg, q4k_weight* wu, q4k_weight* wd, const float* norm_w, float eps, const void* x, void* gate, void* hidden,
             uint32_t m, const uint32_t* query_counts, uint32_t nqueries, uint32_t dtype);

@@ -1887,8 +1887,10 @@ constexpr int kNormRegs = 16;
 
 // RMS norm of one row per workgroup of 512 threads, 8 elements (one 16- or
 // two 16-byte loads) per thread and chunk, the row in registers between the
-// sum of squares and the scaling: a single-element form of 16 dependent loads
-// per thread took 11.3 us for 40 fp16 rows of 4096 and 5.9 us for 5.
+// sum of squares and the scaling, against the general form's 16 single-element
+// loads per thread (rows of 4096, replayed back to back): 40 fp16 rows 6.1 ->
+// 3.3 us, 5 6.0 -> 3.2, 2048 10.2 -> 7.8; fp32 40 rows 5.0 -> 3.4, 2048 13.3 -> 13.5
+// (bandwidth either way).
 constexpr int kNormChunks = 3;
 template <typename T>
 __global__ __launch_bounds__(512) void rms_norm8_kernel(const T* __restrict__ x, const float* __restrict__ w, T* y, int k, float eps, GatherIndex idx,
