@@ -47,6 +47,14 @@ typedef float f4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef _Float16 h4_any_t __attribute__((ext_vector_type(4), aligned(2)));
 typedef _Float16 h8_any_t __attribute__((ext_vector_type(8), aligned(2)));
 
+// The eight waves' sums added in pairs: three roundings of a sum on its way where
+// adding them in turn makes seven, four of them of more than half the total (the
+// RMS norm of rows of 4096 against 64 bits 5.74e-8 in turn, 5.52e-8 so, at the
+// same times).
+__device__ __forceinline__ float sum8_pairs(const float* p) {
+  return ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+}
+
 // Loads 8 consecutive activations as fp32.
 __device__ __forceinline__ void load8(const float* p, float* v) {
   f4_t a = *reinterpret_cast<const f4_any_t*>(p), b = *reinterpret_cast<const f4_any_t*>(p + 4);

@@ -50,12 +50,11 @@ __device__ __forceinline__ void block_max_sum(float& mx, float& ss) {
     red[1][threadIdx.x >> 6] = ss;
   }
   __syncthreads();
-  ss = 0.0f;
+  static_assert(kStageThreads == 8 * 64, "sum8_pairs");
 #pragma unroll
-  for (int w = 0; w < kStageThreads / 64; ++w) {
+  for (int w = 0; w < 8; ++w)
     mx = fmaxf(mx, red[0][w]);
-    ss += red[1][w];
-  }
+  ss = sum8_pairs(red[1]);
 }
 
 // Fused RMS norm of a staged row (native_ops.metal:6-40): the staging
@@ -1923,11 +1922,7 @@ __global__ __launch_bounds__(512) void rms_norm8_kernel(const T* __restrict__ x,
   if ((tid & 63) == 0)
     part[tid >> 6] = ss;
   __syncthreads();
-  float total = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    total += part[i];
-  const float scale = 1.0f / sqrtf(total / (float)k + eps);
+  const float scale = 1.0f / sqrtf(sum8_pairs(part) / (float)k + eps);
   T* yr = y + (size_t)r * k;
 #pragma unroll
   for (int j = 0; j < kNormChunks; ++j) {

@@ -350,15 +350,12 @@ __global__ __launch_bounds__(512) void stage_row_kernel(const InT* __restrict__ 
     red[1][tid >> 6] = ss;
   }
   __syncthreads();
-  ss = 0.0f;
 #pragma unroll
-  for (int w = 0; w < 8; ++w) {
+  for (int w = 0; w < 8; ++w)
     mx = fmaxf(mx, red[0][w]);
-    ss += red[1][w];
-  }
   float r = 1.0f;
   if (NORM) {
-    r = 1.0f / sqrtf(ss / (float)k + eps);
+    r = 1.0f / sqrtf(sum8_pairs(red[1]) / (float)k + eps);
     mx *= r;
   }
   float up, down;
